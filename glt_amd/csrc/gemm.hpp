@@ -86,7 +86,12 @@ struct GemmPlan {
 // form: such a plan must be MFMA-eligible.
 glt_status run_gemm(GemmPlan& plan, hipStream_t st, bool allow_mfma = true);
 bool gemm_mfma_eligible(const GemmPlan& plan);
-// Workgroups of the MFMA kernel's launch for this plan (one per 256 x 256
+// The MFMA kernel for launches that do not fill the chip with 256 x 256 tiles
+// (gemm_kslice.hip): the tile shape to run an MFMA-eligible plan with, or -1
+// for the persistent kernel; and the launch.
+int pick_kslice(const GemmPlan& plan, int cus);
+glt_status run_kslice(GemmPlan& plan, int shape, hipStream_t st);
+// Workgroups of the persistent MFMA kernel's launch for this plan (one per 256 x 256
 // tile, dual: 256 x 128, at most one per CU).
 int gemm_mfma_tiles(const GemmPlan& plan);
 // CUs of the current device (cached per device).

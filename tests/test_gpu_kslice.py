@@ -1,0 +1,67 @@
+"""GPU parity of the K-sliced MFMA GEMM: launches of few tiles, at the edges of
+its tile shapes (32 x 32 to 128 x 256), with reductions whose K-steps do not
+divide evenly over the wavefront groups and their unrolled steps."""
+import numpy as np
+import pytest
+
+from helpers import assert_bf16_budget, draw, make_layer, rel_l2, to_dev, to_np
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [1, 31, 33, 64, 65, 129, 200, 257, 400])
+@pytest.mark.parametrize("K,V", [(64, 2048), (704, 4104), (1088, 16000)])
+def test_head_both_ways(dev, M, K, V):
+    """LM head (bf16 out, K = 1, 11 or 17 steps; V ends inside a tile) and its
+    backward (f32 out, K = V padded to whole steps where V is a multiple of 64,
+    else the strided kernel) against f64. One bf16 rounding; f32 sums of exact
+    products: rel-L2 within 1e-6 per doubling of the number of terms."""
+    import torch
+    from glt_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(M * 7919 + K)
+    x = torch.randn((M, K), generator=g, device="cuda").bfloat16()
+    w = torch.randn((V, K), generator=g, device="cuda").mul_(0.05).bfloat16()
+    y = ops.lm_head_fwd(x, w)
+    assert_bf16_budget(to_np(y), (x.double() @ w.double().t()).cpu().numpy(), q=1, what="logits")
+    if K >= 512:  # K output columns
+        gr = torch.randn((M, V), generator=g, device="cuda").bfloat16()
+        dx = ops.lm_head_bwd(gr, w)
+        assert rel_l2(to_np(dx), (gr.double() @ w.double()).cpu().numpy()) <= 1e-6 * np.log2(V)
+
+
+@pytest.mark.parametrize("M", [7, 40, 70, 130, 300, 520])
+def test_mlp_slices(dev, M):
+    """Forward and backward with an in-place slice over base columns, one with
+    an H offset and an appended one (tiles of two and three K-segments, tiles
+    with none), residual output included."""
+    import torch
+    from glt_amd import ops, synth
+    D, I = 1024, 3008
+    pl = [(64, 192, 0, 1024), (1024, 128, 512, 448), (I, 192, 0, 1024)]
+    N = I + 192 + 64  # the last 64 columns have no segment
+    wg, wu, wd, sl = make_layer(D, I, N, pl, True)
+    dt = torch.bfloat16
+    x = draw((M, D), 100, synth.TID_X, 0, 1, True)
+    dy = draw((M, D), 200, synth.TID_DY, 0, 1, True)
+    base = ops.BaseMLP(to_dev(wg, dt), to_dev(wu, dt), to_dev(wd, dt))
+    gs = [ops.GraftSlice(s["i0"], s["s"], s["h0"], s["h"], *(to_dev(s[p], torch.float32) for p in ("gate", "up", "down")))
+          .pack() for s in sl]
+    xd, dyd = to_dev(x, dt), to_dev(dy, dt)
+    y, g, u, inter = ops.mlp_forward(base, gs, xd, N)
+    dx, grads = ops.mlp_backward(base, gs, xd, dyd, N, g, u, inter)
+    res = xd.clone()
+    ops.mlp_forward(base, gs, xd, N, residual=res)
+    torch.cuda.synchronize()
+    rg, ru, ri, ry = O.mlp_fwd(x, wg, wu, wd, N, sl)
+    rdx, rgr = O.mlp_bwd(x, wg, wu, wd, N, sl, rg, ru, ri, dy)
+    for name, t, r, q in (("g", g, rg, 2), ("u", u, ru, 2), ("inter", inter, ri, 3), ("y", y, ry, 4), ("dx", dx, rdx, 4)):
+        assert_bf16_budget(to_np(t), r, q=q, what=name)
+    assert torch.equal(res, (xd.float() + y.float()).bfloat16())  # the rounded output, added and rounded
+    assert np.all(to_np(inter)[:, I + 192:] == 0)
+    # over few tokens the roundings of the saved operand do not average out:
+    # inter carries three (gate, up, their product), dgate / dup four (gate,
+    # up, the gradient of both and its own), and its sum with exact x or dy none
+    for j in range(len(pl)):
+        for p in range(3):
+            assert_bf16_budget(to_np(grads[j][p]), rgr[j][p], q=4, what=f"slice {j} projection {p}")
