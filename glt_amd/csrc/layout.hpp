@@ -23,6 +23,9 @@ struct T16Job {
   void* dst;
   int rows, cols;
   int64_t src_ld;
+  // Output pitch, 0 for rows. Rows rounded up to 64 take a source whose last
+  // tile is ragged: the columns past `rows` become zero.
+  int64_t dst_ld = 0;
 };
 glt_status transpose_batch(const T16Job* jobs, int n, int dtype, hipStream_t st);
 
@@ -63,13 +66,13 @@ inline int64_t prep_bytes(int I, int D) { return prep_offset(I, D, 6) * 2; }
 // src[r*ld + k] (transposed = false) or src[k*ld + r] (transposed = true);
 // src_dtype GLT_DTYPE_BF16 or GLT_DTYPE_F32 (rounded to bf16, RNE).
 // Two transposed operands of one shape (B[n][k] = src[k][n], rows x K) into
-// the fragment layout in one launch when they are bf16 in whole 64 x 64
-// tiles, else two shuffle_b calls.
+// the fragment layout in one launch when they are bf16 and rows is a multiple
+// of 64 (K may be ragged), else two shuffle_b calls.
 glt_status shuffle_b_tr_pair(const void* src0, const void* src1, int src_dtype, int64_t ld, int rows, int K,
                             uint16_t* dst0, uint16_t* dst1, hipStream_t st);
 glt_status shuffle_b(const void* src, int src_dtype, int64_t ld, bool transposed, int rows, int K, uint16_t* dst,
                      hipStream_t st);
-// shuffle_b_tr_pair for a bf16 src0 and an f32 src1 (whole 64 x 64 tiles,
+// shuffle_b_tr_pair for a bf16 src0 and an f32 src1 (rows a multiple of 64,
 // 16-byte aligned): src1 is rounded to bf16 (RNE) and its row-major bf16
 // copy is written to rm1 in the same pass.
 bool shuffle_tr_pair_f32_ok(const void* src0, const float* src1, int64_t ld, int rows, int K, const void* dst0,

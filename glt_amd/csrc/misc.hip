@@ -126,7 +126,7 @@ struct T16Batch {
   const uint16_t* src[kMaxT16Jobs];
   uint16_t* dst[kMaxT16Jobs];
   int rows[kMaxT16Jobs], cols[kMaxT16Jobs];
-  int64_t ld[kMaxT16Jobs];
+  int64_t ld[kMaxT16Jobs], dst_ld[kMaxT16Jobs];
 };
 
 __global__ void __launch_bounds__(256) transpose16_kernel(const T16Batch bt) {
@@ -140,13 +140,15 @@ __global__ void __launch_bounds__(256) transpose16_kernel(const T16Batch bt) {
   const uint16_t* __restrict__ src = bt.src[j];
   uint16_t* __restrict__ dst = bt.dst[j];
   const int rows = bt.rows[j], tcols = bt.cols[j] / 64;
-  const int64_t src_ld = bt.ld[j];
+  const int64_t src_ld = bt.ld[j], dst_ld = bt.dst_ld[j];
   const int r0 = (int)(tile / tcols) * 64, c0 = (int)(tile % tcols) * 64;
   const int cb = lane & 7, kb = lane >> 3;
   u32x4 in[8];
 #pragma unroll
   for (int r = 0; r < 8; ++r)
-    in[r] = *reinterpret_cast<const u32x4*>(src + (int64_t)(r0 + 8 * kb + r) * src_ld + c0 + 8 * cb);
+    in[r] = r0 + 8 * kb + r < rows
+                ? *reinterpret_cast<const u32x4*>(src + (int64_t)(r0 + 8 * kb + r) * src_ld + c0 + 8 * cb)
+                : u32x4{0u, 0u, 0u, 0u};  // past a ragged source
 #pragma unroll
   for (int c = 0; c < 8; ++c) {
     // output word w of column c = (row 2w, row 2w+1) halves c & 1 of word c / 2
@@ -154,13 +156,16 @@ __global__ void __launch_bounds__(256) transpose16_kernel(const T16Batch bt) {
     u32x4 o;
 #pragma unroll
     for (int w = 0; w < 4; ++w) o[w] = __builtin_amdgcn_perm(in[2 * w + 1][c >> 1], in[2 * w][c >> 1], sel);
-    *reinterpret_cast<u32x4*>(dst + (int64_t)(c0 + 8 * cb + c) * rows + r0 + 8 * kb) = o;
+    *reinterpret_cast<u32x4*>(dst + (int64_t)(c0 + 8 * cb + c) * dst_ld + r0 + 8 * kb) = o;
   }
 }
 
-static bool t16_ok(const void* src, const void* dst, int rows, int cols, int64_t src_ld) {
-  const bool al = ((reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(dst)) & 15) == 0;
-  return al && rows % 64 == 0 && cols % 64 == 0 && src_ld % 8 == 0;
+// every tile's 16-byte pieces are aligned and inside dst (its pitch holds
+// the rows rounded up to 64)
+static bool t16_ok(const T16Job& J) {
+  const bool al = ((reinterpret_cast<uintptr_t>(J.src) | reinterpret_cast<uintptr_t>(J.dst)) & 15) == 0;
+  const int64_t ld = J.dst_ld ? J.dst_ld : J.rows;
+  return al && ld % 8 == 0 && ld >= cdiv(J.rows, 64) * 64 && J.cols % 64 == 0 && J.src_ld % 8 == 0;
 }
 
 glt_status transpose_any(const void* src, void* dst, int rows, int cols, int64_t src_ld, int dtype,
@@ -173,7 +178,7 @@ glt_status transpose16_batch(const T16Job* jobs, int n, hipStream_t st) {
   int64_t tiles = 0;
   for (int j = 0; j < n; ++j) {
     const T16Job& J = jobs[j];
-    GLT_CHECK(t16_ok(J.src, J.dst, J.rows, J.cols, J.src_ld), GLT_ERR_SHAPE,
+    GLT_CHECK(t16_ok(J), GLT_ERR_SHAPE,
               "transpose16_batch: job %d is not whole aligned 64 x 64 tiles", j);
     bt.tile0[j] = tiles;
     bt.src[j] = static_cast<const uint16_t*>(J.src);
@@ -181,7 +186,8 @@ glt_status transpose16_batch(const T16Job* jobs, int n, hipStream_t st) {
     bt.rows[j] = J.rows;
     bt.cols[j] = J.cols;
     bt.ld[j] = J.src_ld;
-    tiles += (int64_t)(J.rows / 64) * (J.cols / 64);
+    bt.dst_ld[j] = J.dst_ld ? J.dst_ld : J.rows;
+    tiles += cdiv(J.rows, 64) * (J.cols / 64);
   }
   bt.tile0[n] = tiles;
   if (tiles == 0) return GLT_OK;
@@ -193,9 +199,11 @@ glt_status transpose16_batch(const T16Job* jobs, int n, hipStream_t st) {
 
 glt_status transpose_batch(const T16Job* jobs, int n, int dtype, hipStream_t st) {
   bool fast = dtype == GLT_DTYPE_BF16;
-  for (int j = 0; fast && j < n; ++j) fast = t16_ok(jobs[j].src, jobs[j].dst, jobs[j].rows, jobs[j].cols, jobs[j].src_ld);
+  for (int j = 0; fast && j < n; ++j) fast = t16_ok(jobs[j]);
   if (fast) return transpose16_batch(jobs, n, st);
   for (int j = 0; j < n; ++j) {
+    GLT_CHECK(!jobs[j].dst_ld || jobs[j].dst_ld == jobs[j].rows, GLT_ERR_UNSUPPORTED,
+              "transpose_batch: job %d has an output pitch and is not bf16 in aligned 64-column tiles", j);
     const glt_status s = transpose_any(jobs[j].src, jobs[j].dst, jobs[j].rows, jobs[j].cols, jobs[j].src_ld, dtype, st);
     if (s != GLT_OK) return s;
   }
@@ -207,8 +215,8 @@ static glt_status launch_transpose(const Tin* src, Tout* dst, int rows, int cols
                                    hipStream_t st) {
   if (rows == 0 || cols == 0) return GLT_OK;
   if constexpr (sizeof(Tin) == 2 && sizeof(Tout) == 2) {
-    if (t16_ok(src, dst, rows, cols, src_ld)) {
-      const T16Job job{src, dst, rows, cols, src_ld};
+    const T16Job job{src, dst, rows, cols, src_ld};
+    if (t16_ok(job)) {
       return transpose16_batch(&job, 1, st);
     }
   }

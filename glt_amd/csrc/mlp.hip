@@ -161,9 +161,19 @@ struct BwdLayout {
   bool wgrad_mfma, dy_f32;
 };
 
-// The weight gradients reduce over the M tokens; on the MFMA kernel that K
-// must be a multiple of 64 as well.
-static bool wgrad_uses_mfma(const glt_mlp_desc* d) { return mlp_uses_mfma(d) && d->M % 64 == 0; }
+// The weight gradients reduce over the M tokens. That K is a whole number of
+// 64-token steps on the MFMA kernel: the operands are laid out with zeros
+// after the last token (1999 tokens, S = 1024, H = 4096: 1617 us on the
+// strided kernel, which took every ragged M, 54 this way).
+static int64_t wgrad_k(const glt_mlp_desc* d) { return shuf_k(d->M); }
+// (the operands' 31-bit offsets hold that many tokens; more run strided)
+static bool wgrad_uses_mfma(const glt_mlp_desc* d) {
+  if (!mlp_uses_mfma(d)) return false;
+  int64_t rows = d->D;
+  if (d->flags & GLT_MLP_EXPLICIT)
+    for (int j = 0; j < d->n_slices; ++j) rows = std::max<int64_t>(rows, d->slices[j].s);
+  return (rows + 256) * wgrad_k(d) * 2 < (int64_t)kOob;
+}
 
 static BwdLayout bwd_layout(const glt_mlp_desc* d) {
   BwdLayout L{};
@@ -191,7 +201,7 @@ static BwdLayout bwd_layout(const glt_mlp_desc* d) {
     L.dyt = off; off += align256((size_t)shuf_elems(d->D, d->M) * 2);
     L.slice0 = off;
     size_t per = 0;
-    for (int j = 0; j < d->n_slices; ++j) per = std::max(per, 3 * align256((size_t)d->slices[j].s * d->M * es));
+    for (int j = 0; j < d->n_slices; ++j) per = std::max(per, 3 * align256((size_t)d->slices[j].s * wgrad_k(d) * es));
     L.slice_stride = per;
     off += per * (size_t)d->n_slices;
   }
@@ -456,6 +466,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
     uint16_t* DYS = reinterpret_cast<uint16_t*>(W + L.dyt);
     if (!operands_laid_out && (s = shuffle_b_tr_pair(x, dy, dt, D, D, M, XS, DYS, st)) != GLT_OK) return s;
     const size_t es = esize(dt);
+    const int64_t Mk = wgrad_k(d);
     // every slice transpose first, batched into few launches
     {
       T16Job jobs[kMaxT16Jobs];
@@ -464,14 +475,14 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
         const glt_graft_slice& sl = d->slices[j];
         const glt_graft_grads& gr = grads[j];
         char* base = W + L.slice0 + (size_t)j * L.slice_stride;
-        const size_t blk = align256((size_t)sl.s * M * es);
+        const size_t blk = align256((size_t)sl.s * Mk * es);
         const char* srcs[3] = {static_cast<const char*>(dg), static_cast<const char*>(du),
                                static_cast<const char*>(inter)};
         const float* outs[3] = {gr.gate, gr.up, gr.down};
         const float* mast[3] = {sl.master_gate, sl.master_up, sl.master_down};
         for (int p = 0; p < 3; ++p) {
           if (!outs[p] || !mast[p]) continue;
-          jobs[nj++] = T16Job{srcs[p] + (size_t)sl.i_start * es, base + p * blk, M, sl.s, (int64_t)N};
+          jobs[nj++] = T16Job{srcs[p] + (size_t)sl.i_start * es, base + p * blk, M, sl.s, (int64_t)N, Mk};
           if (nj == kMaxT16Jobs) {
             if ((s = transpose_batch(jobs, nj, dt, st)) != GLT_OK) return s;
             nj = 0;
@@ -488,7 +499,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
       const glt_graft_slice& sl = d->slices[j];
       const glt_graft_grads& gr = grads[j];
       char* base = W + L.slice0 + (size_t)j * L.slice_stride;
-      const size_t blk = align256((size_t)sl.s * M * es);
+      const size_t blk = align256((size_t)sl.s * Mk * es);
       float* outs[3] = {gr.gate, gr.up, gr.down};
       const float* mast[3] = {sl.master_gate, sl.master_up, sl.master_down};
       for (int p = 0; p < 3; ++p) {
@@ -503,7 +514,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
         }
         // B row of output column h is row h0 + h of the shuffled x / dy
         plan.add_problem(prob(sl.s, sl.h, EPI_STORE, true, outs[p], nullptr, nullptr, sl.h));
-        plan.add_seg(nt_seg(AT, M, 0, M, 0, sl.h, p < 2 ? XS : DYS, M, -sl.h_start));
+        plan.add_seg(nt_seg(AT, Mk, 0, (int)Mk, 0, sl.h, p < 2 ? XS : DYS, Mk, -sl.h_start));
       }
     }
     // The weight-gradient launch has few tiles (3 per slice and 256 x 256

@@ -65,3 +65,47 @@ def test_mlp_slices(dev, M):
     for j in range(len(pl)):
         for p in range(3):
             assert_bf16_budget(to_np(grads[j][p]), rgr[j][p], q=4, what=f"slice {j} projection {p}")
+
+
+@pytest.mark.parametrize("M", [1, 63, 65, 191, 1000])
+def test_ragged_weight_gradients(dev, M):
+    """Token counts off the 64-token steps of the weight-gradient GEMM, whose
+    operands are then padded with zeros: gradients of a slice with an H offset
+    and an appended one against f64 sums of the saved activations, from a bf16
+    and an f32 upstream gradient (the same bits: the values are bf16)."""
+    import torch
+    from glt_amd import ops
+    D, I = 512, 1024
+    pl = [(128, 192, 64, 384), (I, 128, 0, 512)]
+    N = I + 128
+    wg, wu, wd, sl = make_layer(D, I, N, pl, True)
+    dt = torch.bfloat16
+    base = ops.BaseMLP(to_dev(wg, dt), to_dev(wu, dt), to_dev(wd, dt))
+    gs = [ops.GraftSlice(s["i0"], s["s"], s["h0"], s["h"], *(to_dev(s[p], torch.float32) for p in ("gate", "up", "down")))
+          .pack() for s in sl]
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, D), generator=g, device="cuda").to(dt)
+    dy = torch.randn((M, D), generator=g, device="cuda").to(dt)
+    y, gp, up, inter = ops.mlp_forward(base, gs, x, N)
+    nbytes = ops.mlp_backward_workspace(base, gs, M, N) + 2 * M * D + 512  # dy f32: its bf16 copy too
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")     # stale NaN bits in the padding
+    dx, grads = ops.mlp_backward(base, gs, x, dy, N, gp, up, inter, workspace=ws)
+    dx32, grads32 = ops.mlp_backward(base, gs, x, dy.float(), N, gp, up, inter, workspace=ws)
+    assert torch.equal(dx, dx32)
+    dg, du = ops.gate_up_bwd((dy.float() @ torch.cat([base.down.float(), torch.zeros(D, 128, device="cuda")], 1)
+                              + _graft_rows(gs, dy, N)), gp, up)
+    for j, s in enumerate(gs):
+        cols, hs = slice(s.i_start, s.i_start + s.s), slice(s.h_start, s.h_start + s.h)
+        for p, (a, b) in enumerate(((dg, x), (du, x), (inter, dy))):
+            ref = (a[:, cols].double().t() @ b[:, hs].double()).cpu().numpy()
+            # dgate / dup enter the sums rounded to bf16, inter as saved
+            assert_bf16_budget(to_np(grads[j][p]), ref, q=1, what=f"slice {j} projection {p}")
+            assert torch.equal(grads[j][p], grads32[j][p])
+
+
+def _graft_rows(gs, dy, N):
+    import torch
+    out = torch.zeros((dy.shape[0], N), device="cuda")
+    for s in gs:
+        out[:, s.i_start:s.i_start + s.s] += dy[:, s.h_start:s.h_start + s.h].float() @ s.down.bfloat16().float().t()
+    return out
