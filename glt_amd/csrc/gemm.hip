@@ -1,5 +1,5 @@
-// Segment-list GEMM kernels: the gfx950 bf16 MFMA kernel and the strided
-// generic kernel (f32 path, unaligned shapes, graft-GEMM probes).
+// Segment-list GEMM: the persistent gfx950 bf16 MFMA kernel, and the choice
+// between it, the K-sliced kernel and the strided one.
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
@@ -585,74 +585,6 @@ __global__ void __launch_bounds__(256, 1) gemm_mfma_kernel(const GArgs args) {
   __builtin_amdgcn_s_waitcnt(vmcnt_enc(0));
 }
 
-// =========================================================================
-// Generic strided kernel: 64x64 output tile (dual: 64 gate + 64 up columns),
-// K-step 16, operands converted to f32 on load, f32 FMA accumulation.
-// =========================================================================
-template <int KIND>
-__device__ __forceinline__ float ld_kind(const void* p, int64_t i) {
-  if constexpr (KIND == LD_BF16) return bf16_to_f32(static_cast<const uint16_t*>(p)[i]);
-  else if constexpr (KIND == LD_F32) return static_cast<const float*>(p)[i];
-  else return bf16_to_f32(f32_to_bf16(static_cast<const float*>(p)[i]));
-}
-
-template <int LA, int LB, typename TO, int MODE, bool DUAL>
-__global__ void __launch_bounds__(256) gemm_generic_kernel(const GArgs args) {
-  constexpr int BM = 64, BN = 64, BK = 16, NB = DUAL ? 2 : 1;
-  __shared__ float As[BK][BM + 1];
-  __shared__ float Bs[NB][BK][BN + 1];
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  int tm, tn;
-  const int pi = locate_tile(args, blockIdx.x, tm, tn);
-  const GProb& P = args.p[pi];
-  const int m0 = tm * BM, n0 = tn * BN;
-  float acc[NB][4][4] = {};
-  for (int s = P.seg0; s < P.seg0 + P.nseg; ++s) {
-    const GSeg& S = args.s[s];
-    if (!seg_hits(S, P, n0, BN)) continue;
-    const int nhi = min(S.n_hi, P.N);
-    for (int k0 = 0; k0 < S.K; k0 += BK) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int e = tid + 256 * q, r = e >> 4, kk = e & 15;
-        const int m = m0 + r, k = k0 + kk;
-        As[kk][r] = (m < P.M && k < S.K) ? ld_kind<LA>(S.A, (int64_t)m * S.lda + (int64_t)(S.a_col + k) * S.a_ks) : 0.f;
-#pragma unroll
-        for (int h = 0; h < NB; ++h) {
-          const void* B = h ? S.B1 : S.B0;
-          const int64_t ld = h ? S.ldb1 : S.ldb0;
-          const int r0 = h ? S.b1_row0 : S.b0_row0;
-          const int n = n0 + r;
-          Bs[h][kk][r] = (B && n >= S.n_lo && n < nhi && k < S.K)
-                             ? ld_kind<LB>(B, (int64_t)(n - r0) * ld + (int64_t)k * S.b_ks)
-                             : 0.f;
-        }
-      }
-      __syncthreads();
-#pragma unroll
-      for (int kk = 0; kk < BK; ++kk) {
-        float a[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a[i] = As[kk][tr + 16 * i];
-#pragma unroll
-        for (int h = 0; h < NB; ++h)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float b = Bs[h][kk][tc + 16 * j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[h][i][j] = fmaf(a[i], b, acc[h][i][j]);
-          }
-      }
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-      epilogue<TO, MODE>(P, m0 + tr + 16 * i, n0 + tc + 16 * j, acc[0][i][j], DUAL ? acc[NB - 1][i][j] : 0.f);
-}
-
 // ------------------------------------------------------------------ host
 static bool al16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
@@ -728,13 +660,6 @@ static glt_status launch_mfma(const GArgs& a, hipStream_t st, const char* label)
   const int grid = a.total_tiles < cus ? a.total_tiles : cus;
   GLT_LAUNCH(label, fn, dim3(grid), dim3(256), kMfmaLds, st, a);
   GLT_LAUNCH_CHECK("gemm_mfma");
-  return GLT_OK;
-}
-
-template <int LA, int LB, typename TO, int MODE, bool DUAL>
-static glt_status launch_generic(const GArgs& a, hipStream_t st, const char* label) {
-  GLT_LAUNCH(label, (gemm_generic_kernel<LA, LB, TO, MODE, DUAL>), dim3(a.total_tiles), dim3(256), 0, st, a);
-  GLT_LAUNCH_CHECK("gemm_generic");
   return GLT_OK;
 }
 
@@ -817,57 +742,34 @@ glt_status run_gemm(GemmPlan& plan, hipStream_t st, bool allow_mfma) {
     const int shape = pick_kslice(plan, cus);
     if (shape >= 0) return run_kslice(plan, shape, st);
   }
-  const int bm = mfma ? kBM : 64;
-  const int bn = mfma ? (plan.dual ? 128 : 256) : 64;
+  if (!mfma) {
+    GLT_CHECK(plan.b_kind != LD_SHUF && plan.a_kind != LD_SHUF, GLT_ERR_UNSUPPORTED,
+              "run_gemm(%s): shuffled operand on a shape the MFMA kernel does not take", plan.label);
+    return run_strided(plan, st);
+  }
+  const int bn = plan.dual ? 128 : 256;
   const int mode = a.p[0].mode;
   const int of32 = a.p[0].out_f32;
   int tiles = 0;
   for (int p = 0; p < a.nprob; ++p) {
     GProb& P = a.p[p];
     GLT_CHECK(P.mode == mode && P.out_f32 == of32, GLT_ERR_INVALID_ARG, "run_gemm: mixed epilogues in one launch");
-    P.tiles_m = (int)cdiv(P.M, bm);
+    P.tiles_m = (int)cdiv(P.M, kBM);
     P.tiles_n = (int)cdiv(P.N, bn);
     P.tile_begin = tiles;
     tiles += P.tiles_m * P.tiles_n;
   }
   a.total_tiles = tiles;
   if (tiles == 0) return GLT_OK;
-  if (mfma) {
-    if (mode == EPI_SILU && plan.dual) return launch_mfma<uint16_t, EPI_SILU, true>(a, st, plan.label);
-    if (mode == EPI_DGDU && !plan.dual) return launch_mfma<uint16_t, EPI_DGDU, false>(a, st, plan.label);
-    if (mode == EPI_STORE && !plan.dual)
-      return of32 ? launch_mfma<float, EPI_STORE, false>(a, st, plan.label)
-                  : launch_mfma<uint16_t, EPI_STORE, false>(a, st, plan.label);
-    if (mode == EPI_RESID && !plan.dual)
-      return of32 ? launch_mfma<float, EPI_RESID, false>(a, st, plan.label)
-                  : launch_mfma<uint16_t, EPI_RESID, false>(a, st, plan.label);
-    set_error("run_gemm: no MFMA kernel for mode %d dual %d", mode, (int)plan.dual);
-    return GLT_ERR_UNSUPPORTED;
-  }
-  const int la = plan.a_kind, lb = plan.b_kind;
-  GLT_CHECK(lb != LD_SHUF && la != LD_SHUF, GLT_ERR_UNSUPPORTED,
-            "run_gemm(%s): shuffled operand on a shape the MFMA kernel does not take", plan.label);
-#define GLT_GEN(LA_, LB_, TO_, MODE_, DUAL_)                                                     \
-  if (la == LA_ && lb == LB_ && (sizeof(TO_) == 4) == (of32 != 0) && mode == MODE_ && plan.dual == DUAL_) \
-    return launch_generic<LA_, LB_, TO_, MODE_, DUAL_>(a, st, plan.label);
-  // f32 path
-  GLT_GEN(LD_F32, LD_F32, float, EPI_STORE, false)
-  GLT_GEN(LD_F32, LD_F32, float, EPI_RESID, false)
-  GLT_GEN(LD_F32, LD_F32, float, EPI_SILU, true)
-  GLT_GEN(LD_F32, LD_F32, float, EPI_DGDU, false)
-  // bf16 path on shapes the MFMA kernel does not take
-  GLT_GEN(LD_BF16, LD_BF16, uint16_t, EPI_STORE, false)
-  GLT_GEN(LD_BF16, LD_BF16, uint16_t, EPI_RESID, false)
-  GLT_GEN(LD_BF16, LD_BF16, float, EPI_STORE, false)
-  GLT_GEN(LD_BF16, LD_BF16, uint16_t, EPI_SILU, true)
-  GLT_GEN(LD_BF16, LD_BF16, uint16_t, EPI_DGDU, false)
-  // graft-GEMM probes (f32 operands rounded to bf16 on load)
-  GLT_GEN(LD_BF16, LD_F32_AS_BF16, float, EPI_STORE, false)
-  GLT_GEN(LD_F32_AS_BF16, LD_BF16, float, EPI_STORE, false)
-  GLT_GEN(LD_F32_AS_BF16, LD_F32_AS_BF16, float, EPI_STORE, false)
-#undef GLT_GEN
-  set_error("run_gemm: no generic kernel for kinds (%d,%d) out_f32 %d mode %d dual %d", la, lb, of32, mode,
-            (int)plan.dual);
+  if (mode == EPI_SILU && plan.dual) return launch_mfma<uint16_t, EPI_SILU, true>(a, st, plan.label);
+  if (mode == EPI_DGDU && !plan.dual) return launch_mfma<uint16_t, EPI_DGDU, false>(a, st, plan.label);
+  if (mode == EPI_STORE && !plan.dual)
+    return of32 ? launch_mfma<float, EPI_STORE, false>(a, st, plan.label)
+                : launch_mfma<uint16_t, EPI_STORE, false>(a, st, plan.label);
+  if (mode == EPI_RESID && !plan.dual)
+    return of32 ? launch_mfma<float, EPI_RESID, false>(a, st, plan.label)
+                : launch_mfma<uint16_t, EPI_RESID, false>(a, st, plan.label);
+  set_error("run_gemm: no MFMA kernel for mode %d dual %d", mode, (int)plan.dual);
   return GLT_ERR_UNSUPPORTED;
 }
 

@@ -81,8 +81,8 @@ struct GemmPlan {
 
 // Runs the plan: the gfx950 MFMA kernel when A is bf16 row-major (16-byte
 // aligned rows), B is shuffled (LD_SHUF, 32-aligned row ranges) and every K
-// is a multiple of 64; otherwise the strided generic kernel (f32 path,
-// tiny/unaligned shapes, transposed probes). A shuffled B has no generic
+// is a multiple of 64; otherwise the strided kernel (gemm_strided.hip: f32 path,
+// tiny/unaligned shapes, transposed probes). A shuffled B has no strided
 // form: such a plan must be MFMA-eligible.
 glt_status run_gemm(GemmPlan& plan, hipStream_t st, bool allow_mfma = true);
 bool gemm_mfma_eligible(const GemmPlan& plan);
@@ -91,6 +91,8 @@ bool gemm_mfma_eligible(const GemmPlan& plan);
 // for the persistent kernel; and the launch.
 int pick_kslice(const GemmPlan& plan, int cus);
 glt_status run_kslice(GemmPlan& plan, int shape, hipStream_t st);
+// Any plan without a shuffled operand, on the strided f32-MFMA kernel.
+glt_status run_strided(GemmPlan& plan, hipStream_t st);
 // Workgroups of the persistent MFMA kernel's launch for this plan (one per 256 x 256
 // tile, dual: 256 x 128, at most one per CU).
 int gemm_mfma_tiles(const GemmPlan& plan);

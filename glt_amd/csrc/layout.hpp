@@ -39,7 +39,7 @@ inline int64_t shuf_elems(int64_t rows, int64_t k) { return shuf_rows(rows) * sh
 // Packed bf16 mirror of one graft slice (glt_graft_slice.packed), six
 // orientations q = 2*proj + transposed (proj gate, up, down; [S,H] or
 // [H,S]): first row-major, 6*S*H elements in the order gate, gate^T, up,
-// up^T, down, down^T (read by the generic kernel), then, 256-byte aligned,
+// up^T, down, down^T (read by the strided kernel), then, 256-byte aligned,
 // the same six in the shuffled layout (read by the MFMA kernel).
 inline int64_t packed_shuf_base(int S, int H) { return ((int64_t)6 * S * H + 127) / 128 * 128; }
 inline int64_t packed_shuf_offset(int S, int H, int q) {

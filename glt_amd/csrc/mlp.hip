@@ -33,7 +33,7 @@ static const uint16_t* prep(const glt_mlp_desc* d, const glt_base_weights* w, in
 // The bf16 MLP runs on the MFMA kernel when every K is a multiple of 64,
 // every output column range and every operand row offset is 32-aligned
 // (whole shuffled B blocks) and the activation rows are 16-byte aligned;
-// other shapes (and the f32 path) take the strided generic kernel.
+// other shapes (and the f32 path) take the strided kernel.
 static bool mlp_uses_mfma(const glt_mlp_desc* d) {
   if (d->dtype != GLT_DTYPE_BF16) return false;
   if (d->D % 64 || d->I % 64 || d->N % 8) return false;
@@ -543,7 +543,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
     }
     return gs;
   }
-  // strided (generic) form: A(s, t) = src[t*N + i0 + s], B(h, t) = src2[t*D + h0 + h]
+  // strided form: A(s, t) = src[t*N + i0 + s], B(h, t) = src2[t*D + h0 + h]
   GemmPlan plan;
   plan.label = "wgrad";
   plan.a_kind = plan.b_kind = kind;
