@@ -266,50 +266,56 @@ __device__ __forceinline__ void chunk_range(int V, int c, int& v0, int& v1) {
   v1 = min(V, v0 + L);
 }
 
-// The reference hash's passes cut every row into kHashChunks chunks of
-// ceil(V / kHashChunks) logits rounded up to a multiple of 8 (16-byte chunk
-// starts in rows that start on 16 bytes; the last chunks shorter or empty).
-// Any cut gives the same hash. (64 chunks per row, 4x the threads, measured
-// 2 % slower over the three passes at 16384 x 128256: the passes are bound
-// by their arithmetic, not by the chunk walks' load latency.)
-constexpr int kHashChunks = 16;
+// The reference hash's passes cut every row into 2^shift chunks of
+// ceil(V / 2^shift) logits rounded up to a multiple of 8 (the last chunks
+// shorter or empty); any cut gives the same hash. One thread walks one chunk,
+// so the cut sets the threads: about kHashThreads of them, four wavefronts per
+// SIMD (16 chunks per row whatever the rows left half the SIMDs idle at 2048
+// rows: 1.29 ms for the two nibble passes, 0.31 this way, half of that from the
+// eight runs instead of sixteen), between 16 chunks per row and 1024.
+constexpr int64_t kHashThreads = 262144;
+__host__ __device__ inline int hash_shift(int64_t rows) {
+  int sh = 4;
+  while (sh < 10 && (rows << (sh + 1)) <= kHashThreads) ++sh;
+  return sh;
+}
 
-__device__ __forceinline__ void hash_chunk_range(int V, int c, int& v0, int& v1) {
-  const int L = ((V + kHashChunks - 1) / kHashChunks + 7) & ~7;
-  v0 = min(V, c * L);
+__device__ __forceinline__ void hash_chunk_range(int V, int shift, int c, int& v0, int& v1) {
+  const int L = (((V + (1 << shift) - 1) >> shift) + 7) & ~7;
+  v0 = min((int64_t)V, (int64_t)c * L);
   v1 = min(V, v0 + L);
 }
 
-// Calls f(bits) for the bf16 logits x[v0, v1) in order: eight 16-byte loads
-// in flight per thread when the chunk is aligned, else one element a time.
+// Walks the bf16 logits x[v0, v1) in order, f(bits) for one and f2(word) for
+// two (the first in the low half): eight 16-byte loads in flight per thread,
+// single elements up to the first 16-byte boundary (rows of odd V start off
+// it) and after the last whole piece.
+template <typename F, typename F2>
+__device__ __forceinline__ void walk_chunk(const uint16_t* x, int v0, int v1, F&& f, F2&& f2) {
+  int v = v0;
+  for (; v < v1 && (reinterpret_cast<uintptr_t>(x + v) & 15) != 0; ++v) f((uint32_t)x[v]);
+  for (; v + 64 <= v1; v += 64) {
+    u32x4 q[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const u32x4*>(x + v + 8 * i);
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) f2(q[i][e]);
+  }
+  for (; v + 8 <= v1; v += 8) {
+    const u32x4 q = *reinterpret_cast<const u32x4*>(x + v);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) f2(q[e]);
+  }
+  for (; v < v1; ++v) f((uint32_t)x[v]);
+}
 template <typename F>
 __device__ __forceinline__ void walk_chunk(const uint16_t* x, int v0, int v1, F&& f) {
-  const bool vec = ((reinterpret_cast<uintptr_t>(x + v0) & 15) == 0) && ((v1 - v0) % 8 == 0);
-  if (vec) {
-    int v = v0;
-    for (; v + 64 <= v1; v += 64) {
-      u32x4 q[8];
-#pragma unroll
-      for (int i = 0; i < 8; ++i) q[i] = *reinterpret_cast<const u32x4*>(x + v + 8 * i);
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          f(q[i][e] & 0xFFFFu);
-          f(q[i][e] >> 16);
-        }
-    }
-    for (; v < v1; v += 8) {
-      const u32x4 q = *reinterpret_cast<const u32x4*>(x + v);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        f(q[e] & 0xFFFFu);
-        f(q[e] >> 16);
-      }
-    }
-  } else {
-    for (int v = v0; v < v1; ++v) f((uint32_t)x[v]);
-  }
+  walk_chunk(x, v0, v1, f, [&](uint32_t w) {
+    f(w & 0xFFFFu);
+    f(w >> 16);
+  });
 }
 
 // Row-hash form: one workgroup per 16 rows, 16 threads per row: thread c of
@@ -435,31 +441,33 @@ __global__ void __launch_bounds__(256) eval_row_stats_kernel(const uint16_t* log
       s2 = __builtin_fma(d, d, s2);
     }
   };
-  if ((reinterpret_cast<uintptr_t>(x) & 15) == 0 && V % 8 == 0) {
-    const u32x4* xc = reinterpret_cast<const u32x4*>(x);
-    const int nc = V >> 3;
-    int c = tid;
-    for (; c + 768 < nc; c += 1024) {
-      u32x4 q[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) q[u] = __builtin_nontemporal_load(xc + c + 256 * u);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) add8(q[u]);
+  auto add1 = [&](int v) {
+    const float f = __uint_as_float((uint32_t)x[v] << 16);
+    if (f > m) {
+      se *= __expf(m - f);
+      m = f;
     }
-    for (; c < nc; c += 256) add8(__builtin_nontemporal_load(xc + c));
-  } else {
-    for (int v = tid; v < V; v += 256) {
-      const float f = __uint_as_float((uint32_t)x[v] << 16);
-      if (f > m) {
-        se *= __expf(m - f);
-        m = f;
-      }
-      se += __expf(f - m);
-      const double d = (double)f;
-      s += d;
-      s2 = __builtin_fma(d, d, s2);
-    }
+    se += __expf(f - m);
+    const double d = (double)f;
+    s += d;
+    s2 = __builtin_fma(d, d, s2);
+  };
+  // whole 16-byte pieces from the first boundary of the row; the elements
+  // before it (a row of odd V starts off it) and after the last piece one each
+  const int head = min(V, (int)((16 - (reinterpret_cast<uintptr_t>(x) & 15)) & 15) / 2);
+  const u32x4* xc = reinterpret_cast<const u32x4*>(x + head);
+  const int nc = (V - head) >> 3, tail = head + 8 * nc;
+  int c = tid;
+  for (; c + 768 < nc; c += 1024) {
+    u32x4 q[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) q[u] = __builtin_nontemporal_load(xc + c + 256 * u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) add8(q[u]);
   }
+  for (; c < nc; c += 256) add8(__builtin_nontemporal_load(xc + c));
+  if (tid < head) add1(tid);
+  if (tid < V - tail) add1(tail + tid);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     lse_merge(m, se, __shfl_xor(m, o, 64), __shfl_xor(se, o, 64));
@@ -495,253 +503,147 @@ __global__ void __launch_bounds__(256) eval_row_stats_kernel(const uint16_t* log
 // The reference hashes every f32 logit's four little-endian bytes in (b, t, v)
 // order with one FNV-1a chain, h = (h ^ byte) * P mod 2^64 (grafting.hip:536-546),
 // continued across its eval batches. That chain is computed here exactly, in
-// parallel over the chunks of all rows (chunk k = row k / kHashChunks, part
-// k % kHashChunks),
-// in three passes:
+// parallel over the chunks of all rows (chunk k = part k % 2^shift of row
+// k >> shift), in three passes:
 //  * P is odd, so the low byte of h evolves on its own:
 //    s' = ((s ^ byte) * P) mod 256. Bit j of s' depends only on bits 0..j of
-//    s, so the low nibble is a 16-state chain. Pass 1 runs every chunk from
-//    all 16 low nibbles, giving each chunk's map of 16 nibbles; an ordered
-//    scan of the maps from the start hash's nibble gives every chunk's
-//    starting low nibble.
+//    s, so the low nibble is a 16-state chain; and it depends on bit j itself
+//    only by XOR, so starting states that differ in the nibble's top bit end
+//    differing in exactly that bit: eight runs give the map of 16 states
+//    (Map8). Pass 1 runs every chunk from the eight low nibbles 0..7; the maps
+//    compose in order from the start hash's nibble to every chunk's starting
+//    low nibble.
 //  * Pass 2 does the same for the high nibble of the low byte, each chunk's
-//    16 runs starting from its known low nibble.
+//    eight runs starting from its known low nibble.
 //  * With the low byte s of h known at every step, h ^ byte = h + ((s ^ byte)
 //    - s), so a chunk maps h to h * P^(4 n) + B (n logits). Pass 3 runs every
 //    chunk once from h = its starting low byte s, giving B = h_end - s P^(4n);
 //    the (P^(4n), B) pairs compose in order, h <- h A + B.
 // A bf16 logit widens to f32 bits w << 16: its bytes are 0, 0, lo, hi.
-constexpr uint32_t kP16 = (uint32_t)(kFnvPrime & 0xFFFF);
-constexpr uint32_t kP16sq = (uint32_t)((kFnvPrime * kFnvPrime) & 0xFFFF);
-typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+//
+// Each pass's workgroup (256 consecutive chunks) also composes its maps, and
+// the next pass's forms its chunks' starting states from them, so that between
+// two passes only one small launch runs over the workgroups. Passes 1 and 2
+// issue about 18 instructions per logit and are bound by that: with a factor
+// P^2 carried along a logit is t ^= lo, t *= P, t ^= hi, t *= P^3, two runs per
+// register as 8-bit fields 16 bits apart, which one 24-bit multiply serves (a
+// packed 16-bit multiply needs no masks: 166 against 154 us for 2048 rows of
+// 128256, where the issue of these instructions alone is 124).
+constexpr uint32_t kP8 = (uint32_t)(kFnvPrime & 0xFF);
+constexpr uint64_t kP2 = kFnvPrime * kFnvPrime, kP3 = kP2 * kFnvPrime;
+constexpr uint64_t inverse64(uint64_t a) {  // of an odd a, mod 2^64 (Newton, doubling the correct bits)
+  uint64_t x = a;                           // right in 3 bits
+  for (int i = 0; i < 6; ++i) x *= 2 - a * x;
+  return x;
+}
+constexpr uint64_t kP2Inv = inverse64(kP2);
+static_assert(kP2Inv * kP2 == 1, "inverse of P^2 mod 2^64");
 
-__device__ __forceinline__ uint32_t pk_mul(uint32_t a, uint32_t k) {
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(u16x2, a) * (u16x2){(uint16_t)k, (uint16_t)k});
-}
-
-// Pass 1 in bit planes. Per logit the low nibble goes
-//   s <- ((9 s ^ a) * 3 ^ b) * 3 mod 16   (P mod 16 = 3, a / b: low nibbles of lo / hi)
-// and the 16 runs of a chunk are kept as four 16-bit planes (bit i of plane
-// j = bit j of run i), two chunks of one row per thread in the two halves
-// of each 32-bit plane: 9 s flips bit 3 by bit 0, 3 s = s + 2 s is a ripple
-// carry over the planes, and XOR with a logit's bit is a XOR with that bit
-// spread over the chunk's half. About 19 operations per logit, against 40
-// for 16 runs held as 16-bit integers.
-typedef short s16x2 __attribute__((ext_vector_type(2)));
-struct Planes {
-  uint32_t p0, p1, p2, p3;
-};
-// bit k of each 16-bit half of w, spread over that half (0 or 0xFFFF)
-__device__ __forceinline__ uint32_t half_mask(uint32_t w, int k) {
-  return __builtin_bit_cast(uint32_t, __builtin_bit_cast(s16x2, w << (15 - k)) >> (s16x2){15, 15});
-}
-__device__ __forceinline__ void planes_x3(Planes& P) {
-  const uint32_t c1 = P.p1 & P.p0, t = P.p2 ^ P.p1;
-  const uint32_t c2 = (t & c1) | (~t & P.p2);  // carry into bit 3: majority of p2, p1, c1
-  P.p3 ^= P.p2 ^ c2;
-  P.p2 = t ^ c1;
-  P.p1 ^= P.p0;
-}
-// one logit of each chunk: chunk A's 16 bits in the low half of w, B's high
-__device__ __forceinline__ void planes_step(Planes& P, uint32_t w) {
-  P.p3 ^= P.p0 ^ half_mask(w, 3);  // 9 s, then ^ a
-  P.p0 ^= half_mask(w, 0);
-  P.p1 ^= half_mask(w, 1);
-  P.p2 ^= half_mask(w, 2);
-  planes_x3(P);
-  P.p0 ^= half_mask(w, 8);
-  P.p1 ^= half_mask(w, 9);
-  P.p2 ^= half_mask(w, 10);
-  P.p3 ^= half_mask(w, 11);
-  planes_x3(P);
-}
-// chunk pair kp = chunks 2 kp, 2 kp + 1 (the same row: kHashChunks is even);
-// the second one is never longer than the first
-static_assert(kHashChunks % 2 == 0, "chunk pairs share a row");
-__global__ void __launch_bounds__(256) hash_lo_planes_kernel(const uint16_t* logits, int64_t ld, int64_t chunks, int V,
-                                                             uint64_t* __restrict__ maps) {
-  const int64_t kA = 2 * ((int64_t)blockIdx.x * 256 + threadIdx.x);
-  if (kA >= chunks) return;
-  const uint16_t* x = logits + (kA / kHashChunks) * ld;
-  int a0, a1, b0, b1;
-  hash_chunk_range(V, (int)(kA & (kHashChunks - 1)), a0, a1);
-  hash_chunk_range(V, (int)((kA + 1) & (kHashChunks - 1)), b0, b1);
-  const int na = a1 - a0, nb = b1 - b0;
-  Planes P{0xAAAAAAAAu, 0xCCCCCCCCu, 0xF0F0F0F0u, 0xFF00FF00u};  // run i starts at nibble i
-  auto step2 = [&](uint32_t qa, uint32_t qb) {  // two logits of each chunk, in order
-    planes_step(P, (qa & 0xFFFFu) | (qb << 16));
-    planes_step(P, (qa >> 16) | (qb & 0xFFFF0000u));
-  };
-  int v = 0;
-  const bool vec = ((reinterpret_cast<uintptr_t>(x + a0) | reinterpret_cast<uintptr_t>(x + b0)) & 15) == 0;
-  if (vec) {
-    const u32x4* xa = reinterpret_cast<const u32x4*>(x + a0);
-    const u32x4* xb = reinterpret_cast<const u32x4*>(x + b0);
-    for (; v + 32 <= nb; v += 32) {
-      u32x4 qa[4], qb[4];
+// Map of 16 nibbles f with f(s ^ 8) = f(s) ^ 8: nibble i of the word is f(i),
+// i < 8.
+typedef uint32_t Map8;
+constexpr Map8 kMapIdentity = 0x76543210u;
+__device__ __forceinline__ uint32_t map_apply(Map8 f, uint32_t s) { return ((f >> (4 * (s & 7))) & 15u) ^ (s & 8u); }
+__device__ __forceinline__ Map8 map_then(Map8 f, Map8 g) {  // first f, then g
+  Map8 h = 0;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        qa[u] = xa[(v >> 3) + u];
-        qb[u] = xb[(v >> 3) + u];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) step2(qa[u][e], qb[u][e]);
-    }
-    for (; v + 8 <= nb; v += 8) {
-      const u32x4 qa = xa[v >> 3], qb = xb[v >> 3];
-#pragma unroll
-      for (int e = 0; e < 4; ++e) step2(qa[e], qb[e]);
-    }
-  }
-  for (; v < nb; ++v) planes_step(P, (uint32_t)x[a0 + v] | ((uint32_t)x[b0 + v] << 16));
-  // the rest of chunk A (B ran out): B's half of every plane is kept
-  for (; v < na; ++v) {
-    const Planes Q = P;
-    planes_step(P, (uint32_t)x[a0 + v]);
-    P.p0 = (P.p0 & 0xFFFFu) | (Q.p0 & 0xFFFF0000u);
-    P.p1 = (P.p1 & 0xFFFFu) | (Q.p1 & 0xFFFF0000u);
-    P.p2 = (P.p2 & 0xFFFFu) | (Q.p2 & 0xFFFF0000u);
-    P.p3 = (P.p3 & 0xFFFFu) | (Q.p3 & 0xFFFF0000u);
-  }
-  uint64_t mA = 0, mB = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) {
-    const uint32_t sa = ((P.p0 >> i) & 1u) | (((P.p1 >> i) & 1u) << 1) | (((P.p2 >> i) & 1u) << 2) |
-                        (((P.p3 >> i) & 1u) << 3);
-    const uint32_t sb = ((P.p0 >> (16 + i)) & 1u) | (((P.p1 >> (16 + i)) & 1u) << 1) |
-                        (((P.p2 >> (16 + i)) & 1u) << 2) | (((P.p3 >> (16 + i)) & 1u) << 3);
-    mA |= (uint64_t)sa << (4 * i);
-    mB |= (uint64_t)sb << (4 * i);
-  }
-  maps[kA] = mA;
-  maps[kA + 1] = mB;
-}
-
-// Pass 2: 16 runs of the low-byte chain over chunk k, two per register
-// (16-bit halves; the low byte of a product depends only on the operands'
-// low bytes, so the high bytes may hold anything), run i starting at
-// (i << 4) | the chunk's starting low nibble. maps[k] nibble i = the final
-// high nibble of run i.
-__global__ void __launch_bounds__(256) hash_hi_nibble_kernel(const uint16_t* logits, int64_t ld, int64_t chunks, int V,
-                                                             const uint8_t* __restrict__ start_lo,
-                                                             uint64_t* __restrict__ maps) {
-  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (k >= chunks) return;
-  const uint32_t base = start_lo[k];
-  uint32_t st[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) st[i] = (base | ((2 * i) << 4)) | ((base | ((2 * i + 1) << 4)) << 16);
-  int v0, v1;
-  hash_chunk_range(V, (int)(k & (kHashChunks - 1)), v0, v1);
-  walk_chunk(logits + (k / kHashChunks) * ld, v0, v1, [&](uint32_t w) {
-    const uint32_t lo = (w & 0xFFu) * 0x10001u, hi = (w >> 8) * 0x10001u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) st[i] = pk_mul(pk_mul(pk_mul(st[i], kP16sq) ^ lo, kP16) ^ hi, kP16);
-  });
-  uint64_t m = 0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int hh = 0; hh < 2; ++hh) {
-      const uint32_t v = (st[i] >> (16 * hh)) & 0xFFu;
-      m |= (uint64_t)(v >> 4) << (4 * (2 * i + hh));
-    }
-  maps[k] = m;
-}
-
-// 16-nibble maps: apply, and compose (first f, then g).
-__device__ __forceinline__ uint32_t nib_apply(uint64_t f, uint32_t s) { return (uint32_t)(f >> (4 * s)) & 15u; }
-__device__ __forceinline__ uint64_t nib_compose(uint64_t f, uint64_t g) {
-  uint64_t h = 0;
-#pragma unroll
-  for (int i = 0; i < 16; ++i) h |= (uint64_t)nib_apply(g, nib_apply(f, i)) << (4 * i);
+  for (int i = 0; i < 8; ++i) h |= map_apply(g, (f >> (4 * i)) & 15u) << (4 * i);
   return h;
 }
-constexpr uint64_t kNibIdentity = 0xFEDCBA9876543210ull;
-constexpr int kScanPer = 4, kScanBlock = 256 * kScanPer;  // chunks per scan workgroup
-
-// Ordered scan of the chunk maps, step 1: each workgroup's composition of
-// its kScanBlock maps (in order, by an order-preserving tree in LDS).
-__global__ void __launch_bounds__(256) nib_scan_up_kernel(const uint64_t* __restrict__ maps, int64_t chunks,
-                                                          uint64_t* __restrict__ agg) {
-  __shared__ uint64_t s[256];
+// The composition of the maps of threads 0 .. t-1 (in that order) of the 256
+// threads; *total that of all.
+__device__ __forceinline__ Map8 scan_maps(Map8 f, Map8* lds, Map8* total) {
   const int t = threadIdx.x;
-  uint64_t f = kNibIdentity;
-  for (int i = 0; i < kScanPer; ++i) {
-    const int64_t k = (int64_t)blockIdx.x * kScanBlock + t * kScanPer + i;
-    if (k < chunks) f = nib_compose(f, maps[k]);
-  }
-  s[t] = f;
+  lds[t] = f;
   __syncthreads();
   for (int w = 1; w < 256; w *= 2) {
-    if ((t & (2 * w - 1)) == 0) s[t] = nib_compose(s[t], s[t + w]);
+    const Map8 g = t >= w ? lds[t - w] : kMapIdentity;
+    __syncthreads();
+    f = map_then(g, f);
+    lds[t] = f;
     __syncthreads();
   }
-  if (t == 0) agg[blockIdx.x] = s[0];
+  const Map8 before = t ? lds[t - 1] : kMapIdentity;
+  *total = lds[255];
+  __syncthreads();
+  return before;
 }
 
-// Step 2: the starting nibble of every workgroup, in order from `start`:
-// each thread composes a run of consecutive workgroup maps, thread 0 walks
-// the 256 run maps, and each thread then walks its own run.
-__global__ void __launch_bounds__(256) nib_scan_top_kernel(const uint64_t* __restrict__ agg, int64_t nblocks,
-                                                           uint32_t start, uint8_t* __restrict__ bstart) {
-  __shared__ uint64_t run[256];
-  __shared__ uint8_t rs[256];
+// Pass 1 (HIGH false) and 2 (HIGH true) over 256 chunks: maps[k] of chunk k
+// and agg[block] of the workgroup's chunks in order. Pass 2 first forms its
+// chunks' starting low nibbles from pass 1's maps (lo_maps) and the
+// workgroup's (lo_start), and writes them to start[k].
+template <bool HIGH>
+__global__ void __launch_bounds__(256) hash_nibble_kernel(const uint16_t* logits, int64_t ld, int64_t chunks, int shift,
+                                                          int V, const Map8* __restrict__ lo_maps,
+                                                          const uint8_t* __restrict__ lo_start,
+                                                          uint8_t* __restrict__ start, Map8* __restrict__ maps,
+                                                          Map8* __restrict__ agg) {
+  __shared__ Map8 lds[256];
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const bool in = k < chunks;
+  Map8 total;
+  uint32_t base = 0;
+  if (HIGH) {
+    const Map8 before = scan_maps(in ? lo_maps[k] : kMapIdentity, lds, &total);
+    base = map_apply(before, lo_start[blockIdx.x]);
+    if (in) start[k] = (uint8_t)base;
+  }
+  Map8 f = kMapIdentity;
+  if (in) {
+    // fields 0 and 16 of st[j]: runs 2 j and 2 j + 1 (times P^2; the bits
+    // above each field's 8 are left over)
+    constexpr uint32_t kFields = 0x00FF00FFu;
+    uint32_t st[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t a = HIGH ? base | (2 * j) << 4 : 2 * j, b = HIGH ? base | (2 * j + 1) << 4 : 2 * j + 1;
+      st[j] = (a | b << 16) * (uint32_t)(kP2 & 0xFF);
+    }
+    int v0, v1;
+    hash_chunk_range(V, shift, (int)(k & ((1 << shift) - 1)), v0, v1);
+    auto logit = [&](uint32_t lo, uint32_t hi) {  // each byte in both fields
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        st[j] = ((st[j] ^ lo) & kFields) * kP8;
+        st[j] = ((st[j] ^ hi) & kFields) * (uint32_t)(kP3 & 0xFF);
+      }
+    };
+    walk_chunk(
+        logits + (k >> shift) * ld, v0, v1,
+        [&](uint32_t w) {
+          logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
+        },
+        [&](uint32_t w) {
+          logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
+          logit(__builtin_amdgcn_perm(0u, w, 0x0C020C02u), __builtin_amdgcn_perm(0u, w, 0x0C030C03u));
+        });
+    f = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t s2 = ((st[j] & kFields) * (uint32_t)(kP2Inv & 0xFF)) >> (HIGH ? 4 : 0);
+      f |= ((s2 & 15u) | ((s2 >> 16) & 15u) << 4) << (8 * j);
+    }
+    maps[k] = f;
+  }
+  scan_maps(f, lds, &total);
+  if (threadIdx.x == 0) agg[blockIdx.x] = total;
+}
+
+// Starting nibble of every workgroup's first chunk from the start hash's
+// nibble, in order.
+__global__ void __launch_bounds__(256) hash_starts_kernel(const Map8* __restrict__ agg, int64_t nblocks, uint32_t start,
+                                                          uint8_t* __restrict__ bstart) {
+  __shared__ Map8 lds[256];
   const int t = threadIdx.x;
   const int64_t q = (nblocks + 255) / 256;
   const int64_t b0 = min(nblocks, t * q), b1 = min(nblocks, b0 + q);
-  uint64_t f = kNibIdentity;
-  for (int64_t b = b0; b < b1; ++b) f = nib_compose(f, agg[b]);
-  run[t] = f;
-  __syncthreads();
-  if (t == 0) {
-    uint32_t s = start;
-    for (int i = 0; i < 256; ++i) {
-      rs[i] = (uint8_t)s;
-      s = nib_apply(run[i], s);
-    }
-  }
-  __syncthreads();
-  uint32_t s = rs[t];
+  Map8 f = kMapIdentity, total;
+  for (int64_t b = b0; b < b1; ++b) f = map_then(f, agg[b]);
+  uint32_t s = map_apply(scan_maps(f, lds, &total), start);
   for (int64_t b = b0; b < b1; ++b) {
     bstart[b] = (uint8_t)s;
-    s = nib_apply(agg[b], s);
-  }
-}
-
-// Step 3: every chunk's starting nibble. OR_SHIFT 0 writes it to out[k];
-// 4 ORs it in as the high nibble (out then holds whole starting bytes).
-template <int OR_SHIFT>
-__global__ void __launch_bounds__(256) nib_scan_down_kernel(const uint64_t* __restrict__ maps, int64_t chunks,
-                                                            const uint8_t* __restrict__ bstart,
-                                                            uint8_t* __restrict__ out) {
-  __shared__ uint64_t s[256];
-  __shared__ uint8_t ts[256];
-  const int t = threadIdx.x;
-  uint64_t f = kNibIdentity;
-  for (int i = 0; i < kScanPer; ++i) {
-    const int64_t k = (int64_t)blockIdx.x * kScanBlock + t * kScanPer + i;
-    if (k < chunks) f = nib_compose(f, maps[k]);
-  }
-  s[t] = f;
-  __syncthreads();
-  if (t == 0) {
-    uint32_t st = bstart[blockIdx.x];
-    for (int i = 0; i < 256; ++i) {
-      ts[i] = (uint8_t)st;
-      st = nib_apply(s[i], st);
-    }
-  }
-  __syncthreads();
-  uint32_t st = ts[t];
-  for (int i = 0; i < kScanPer; ++i) {
-    const int64_t k = (int64_t)blockIdx.x * kScanBlock + t * kScanPer + i;
-    if (k >= chunks) break;
-    if (OR_SHIFT == 0) out[k] = (uint8_t)st;
-    else out[k] = (uint8_t)(out[k] | (st << 4));
-    st = nib_apply(maps[k], st);
+    s = map_apply(agg[b], s);
   }
 }
 
@@ -756,23 +658,30 @@ __device__ __forceinline__ Affine affine_then(Affine x, Affine y) { return Affin
 
 // Pass 3: each chunk run once from h = its starting low byte, reduced to one
 // affine map per workgroup of 256 chunks (order-preserving tree).
-__global__ void __launch_bounds__(256) hash_affine_kernel(const uint16_t* logits, int64_t ld, int64_t chunks, int V,
-                                                          const uint8_t* __restrict__ start_byte,
+__global__ void __launch_bounds__(256) hash_affine_kernel(const uint16_t* logits, int64_t ld, int64_t chunks, int shift,
+                                                          int V, const uint8_t* __restrict__ start_lo,
+                                                          const Map8* __restrict__ hi_maps,
+                                                          const uint8_t* __restrict__ hi_start,
                                                           Affine* __restrict__ out) {
   __shared__ uint64_t sa[256], sb[256];
+  __shared__ Map8 lds[256];
   const int t = threadIdx.x;
   const int64_t k = (int64_t)blockIdx.x * 256 + t;
+  Map8 total;
+  const Map8 before = scan_maps(k < chunks ? hi_maps[k] : kMapIdentity, lds, &total);
   Affine f{1, 0};
   if (k < chunks) {
     int v0, v1;
-    hash_chunk_range(V, (int)(k & (kHashChunks - 1)), v0, v1);
-    const uint64_t s0 = start_byte[k];
-    uint64_t h = s0;
-    walk_chunk(logits + (k / kHashChunks) * ld, v0, v1, [&](uint32_t w) {
-      h = fnv_mul(fnv_mul(h));
+    hash_chunk_range(V, shift, (int)(k & ((1 << shift) - 1)), v0, v1);
+    const uint64_t s0 = start_lo[k] | map_apply(before, hi_start[blockIdx.x]) << 4;
+    // h with a factor P^2 carried along, as in the other passes: two 64-bit
+    // multiplications per logit instead of four
+    uint64_t h = s0 * kP2;
+    walk_chunk(logits + (k >> shift) * ld, v0, v1, [&](uint32_t w) {
       h = fnv_mul(h ^ (w & 0xFFu));
-      h = fnv_mul(h ^ (w >> 8));
+      h = (h ^ (w >> 8)) * kP3;
     });
+    h *= kP2Inv;
     // P^(4 n) by squaring
     uint64_t a = 1, p4 = fnv_mul(fnv_mul(fnv_mul(kFnvPrime)));
     for (uint32_t n = (uint32_t)(v1 - v0); n; n >>= 1, p4 *= p4)
@@ -791,6 +700,45 @@ __global__ void __launch_bounds__(256) hash_affine_kernel(const uint16_t* logits
     __syncthreads();
   }
   if (t == 0) out[blockIdx.x] = Affine{sa[0], sb[0]};
+}
+
+// The whole batch from its rows and (exact hash) its workgroups' affine maps:
+// each thread takes a run of consecutive ones, the runs join in order.
+struct EvalTotal {
+  double nll, sum, sumsq;
+  int64_t count;
+  Affine hash;
+};
+__global__ void __launch_bounds__(256) eval_total_kernel(const EvalRow* __restrict__ rows, int64_t R,
+                                                         const Affine* __restrict__ aff, int64_t naff,
+                                                         EvalTotal* __restrict__ out) {
+  __shared__ EvalTotal s[256];
+  const int t = threadIdx.x;
+  EvalTotal v{0.0, 0.0, 0.0, 0, {1, 0}};
+  const int64_t qr = (R + 255) / 256, qa = (naff + 255) / 256;
+  for (int64_t r = t * qr; r < min(R, (t + 1) * qr); ++r) {
+    v.sum += rows[r].sum;
+    v.sumsq += rows[r].sumsq;
+    if (rows[r].scored) {
+      v.nll += rows[r].nll;
+      ++v.count;
+    }
+  }
+  for (int64_t a = t * qa; a < min(naff, (t + 1) * qa); ++a) v.hash = affine_then(v.hash, aff[a]);
+  s[t] = v;
+  __syncthreads();
+  for (int w = 1; w < 256; w *= 2) {
+    if ((t & (2 * w - 1)) == 0) {
+      const EvalTotal o = s[t + w];
+      s[t].nll += o.nll;
+      s[t].sum += o.sum;
+      s[t].sumsq += o.sumsq;
+      s[t].count += o.count;
+      s[t].hash = affine_then(s[t].hash, o.hash);
+    }
+    __syncthreads();
+  }
+  if (t == 0) *out = s[0];
 }
 
 struct ModelWs {
@@ -930,43 +878,28 @@ glt_status glt_model_fwd(const glt_model* m, const int32_t* ids, uint16_t* logit
 namespace glt {
 namespace {
 struct EvalWs {
-  size_t rows, maps, start, agg, bstart, aff, total;
-  int64_t chunks, nscan, naff;
+  size_t rows, maps_lo, maps_hi, start, agg, bstart_lo, bstart_hi, aff, sums, total;
+  int64_t chunks, blocks;
+  int shift;
 };
 EvalWs eval_ws(int64_t R) {
   EvalWs w{};
-  w.chunks = R * kHashChunks;
-  w.nscan = cdiv(w.chunks, kScanBlock);
-  w.naff = cdiv(w.chunks, 256);
+  w.shift = hash_shift(R);
+  w.chunks = R << w.shift;
+  w.blocks = cdiv(w.chunks, 256);
   w.rows = 0;
-  w.maps = up(w.rows + R * sizeof(EvalRow));
-  w.start = up(w.maps + w.chunks * 8);
+  w.maps_lo = up(w.rows + R * sizeof(EvalRow));
+  w.maps_hi = up(w.maps_lo + w.chunks * sizeof(Map8));
+  w.start = up(w.maps_hi + w.chunks * sizeof(Map8));
   w.agg = up(w.start + w.chunks);
-  w.bstart = up(w.agg + w.nscan * 8);
-  w.aff = up(w.bstart + w.nscan);
-  w.total = up(w.aff + w.naff * sizeof(Affine));
+  w.bstart_lo = up(w.agg + w.blocks * sizeof(Map8));
+  w.bstart_hi = up(w.bstart_lo + w.blocks);
+  w.aff = up(w.bstart_hi + w.blocks);
+  w.sums = up(w.aff + w.blocks * sizeof(Affine));
+  w.total = up(w.sums + sizeof(EvalTotal));
   return w;
 }
 
-// Starting nibble of every chunk from the maps (ordered scan, three launches).
-glt_status nib_scan(const EvalWs& w, char* ws, uint32_t start, bool high, hipStream_t st) {
-  const uint64_t* maps = reinterpret_cast<const uint64_t*>(ws + w.maps);
-  uint64_t* agg = reinterpret_cast<uint64_t*>(ws + w.agg);
-  uint8_t* bstart = reinterpret_cast<uint8_t*>(ws + w.bstart);
-  uint8_t* out = reinterpret_cast<uint8_t*>(ws + w.start);
-  GLT_LAUNCH("eval_hash_scan", nib_scan_up_kernel, dim3((unsigned)w.nscan), dim3(256), 0, st, maps, w.chunks, agg);
-  GLT_LAUNCH_CHECK("nib_scan_up");
-  GLT_LAUNCH("eval_hash_scan", nib_scan_top_kernel, dim3(1), dim3(256), 0, st, agg, w.nscan, start, bstart);
-  GLT_LAUNCH_CHECK("nib_scan_top");
-  if (high)
-    GLT_LAUNCH("eval_hash_scan", nib_scan_down_kernel<4>, dim3((unsigned)w.nscan), dim3(256), 0, st, maps, w.chunks,
-               bstart, out);
-  else
-    GLT_LAUNCH("eval_hash_scan", nib_scan_down_kernel<0>, dim3((unsigned)w.nscan), dim3(256), 0, st, maps, w.chunks,
-               bstart, out);
-  GLT_LAUNCH_CHECK("nib_scan_down");
-  return GLT_OK;
-}
 }  // namespace
 }  // namespace glt
 
@@ -992,7 +925,7 @@ glt_status glt_eval_stats(const uint16_t* logits, int64_t ld, const int32_t* ids
             glt_eval_stats_workspace_size(B, T), kAlign);
   const bool exact = hash_mode == GLT_EVAL_HASH_REFERENCE;
   const EvalWs w = eval_ws(R);
-  GLT_CHECK(w.naff < INT32_MAX, GLT_ERR_SHAPE, "glt_eval_stats: %lld rows", (long long)R);
+  GLT_CHECK(w.blocks < INT32_MAX, GLT_ERR_SHAPE, "glt_eval_stats: %lld rows", (long long)R);
   hipStream_t st = as_stream(stream);
   char* ws = static_cast<char*>(workspace);
   EvalRow* rows = reinterpret_cast<EvalRow*>(ws + w.rows);
@@ -1004,27 +937,43 @@ glt_status glt_eval_stats(const uint16_t* logits, int64_t ld, const int32_t* ids
   GLT_LAUNCH_CHECK("eval_rows");
   Affine* aff = reinterpret_cast<Affine*>(ws + w.aff);
   if (exact) {
-    uint64_t* maps = reinterpret_cast<uint64_t*>(ws + w.maps);
+    Map8* maps_lo = reinterpret_cast<Map8*>(ws + w.maps_lo);
+    Map8* maps_hi = reinterpret_cast<Map8*>(ws + w.maps_hi);
+    Map8* agg = reinterpret_cast<Map8*>(ws + w.agg);
     uint8_t* start = reinterpret_cast<uint8_t*>(ws + w.start);
-    const dim3 grid((unsigned)w.naff);
-    GLT_LAUNCH("eval_hash_nibble", hash_lo_planes_kernel, dim3((unsigned)cdiv(w.chunks / 2, 256)), dim3(256), 0, st,
-               logits, ld, w.chunks, V, maps);
+    uint8_t* b_lo = reinterpret_cast<uint8_t*>(ws + w.bstart_lo);
+    uint8_t* b_hi = reinterpret_cast<uint8_t*>(ws + w.bstart_hi);
+    const dim3 grid((unsigned)w.blocks);
+    GLT_LAUNCH("eval_hash_nibble", hash_nibble_kernel<false>, grid, dim3(256), 0, st, logits, ld, w.chunks, w.shift, V,
+               (const Map8*)nullptr, (const uint8_t*)nullptr, (uint8_t*)nullptr, maps_lo, agg);
     GLT_LAUNCH_CHECK("hash_nibble");
-    glt_status s = nib_scan(w, ws, (uint32_t)(hash_in & 15), false, st);
-    if (s != GLT_OK) return s;
-    GLT_LAUNCH("eval_hash_nibble", hash_hi_nibble_kernel, grid, dim3(256), 0, st, logits, ld, w.chunks, V,
-               (const uint8_t*)start, maps);
+    GLT_LAUNCH("eval_hash_scan", hash_starts_kernel, dim3(1), dim3(256), 0, st, agg, w.blocks, (uint32_t)(hash_in & 15),
+               b_lo);
+    GLT_LAUNCH_CHECK("hash_starts");
+    GLT_LAUNCH("eval_hash_nibble", hash_nibble_kernel<true>, grid, dim3(256), 0, st, logits, ld, w.chunks, w.shift, V,
+               maps_lo, b_lo, start, maps_hi, agg);
     GLT_LAUNCH_CHECK("hash_nibble");
-    if ((s = nib_scan(w, ws, (uint32_t)((hash_in >> 4) & 15), true, st)) != GLT_OK) return s;
-    GLT_LAUNCH("eval_hash_affine", hash_affine_kernel, grid, dim3(256), 0, st, logits, ld, w.chunks, V,
-               (const uint8_t*)start, aff);
+    GLT_LAUNCH("eval_hash_scan", hash_starts_kernel, dim3(1), dim3(256), 0, st, agg, w.blocks,
+               (uint32_t)((hash_in >> 4) & 15), b_hi);
+    GLT_LAUNCH_CHECK("hash_starts");
+    GLT_LAUNCH("eval_hash_affine", hash_affine_kernel, grid, dim3(256), 0, st, logits, ld, w.chunks, w.shift, V, start,
+               maps_hi, b_hi, aff);
     GLT_LAUNCH_CHECK("hash_affine");
   }
+  if (exact) {
+    EvalTotal* sums = reinterpret_cast<EvalTotal*>(ws + w.sums);
+    GLT_LAUNCH("eval_total", eval_total_kernel, dim3(1), dim3(256), 0, st, rows, R, aff, w.blocks, sums);
+    GLT_LAUNCH_CHECK("eval_total");
+    EvalTotal h;
+    GLT_CHECK(hipMemcpyAsync(&h, sums, sizeof h, hipMemcpyDeviceToHost, st) == hipSuccess &&
+                  hipStreamSynchronize(st) == hipSuccess,
+              GLT_ERR_HIP, "glt_eval_stats: copy of the results failed");
+    *out = glt_eval_result{h.nll, h.count, h.sum, h.sumsq, hash_in * h.hash.a + h.hash.b};
+    return GLT_OK;
+  }
+  // the rows form chains the row hashes byte by byte, on the host
   std::vector<EvalRow> h((size_t)R);
-  std::vector<Affine> ha(exact ? (size_t)w.naff : 0);
   GLT_CHECK(hipMemcpyAsync(h.data(), rows, (size_t)R * sizeof(EvalRow), hipMemcpyDeviceToHost, st) == hipSuccess &&
-                (!exact || hipMemcpyAsync(ha.data(), aff, ha.size() * sizeof(Affine), hipMemcpyDeviceToHost, st) ==
-                               hipSuccess) &&
                 hipStreamSynchronize(st) == hipSuccess,
             GLT_ERR_HIP, "glt_eval_stats: copy of the results failed");
   uint64_t hash = hash_in;
@@ -1035,13 +984,11 @@ glt_status glt_eval_stats(const uint16_t* logits, int64_t ld, const int32_t* ids
       out->total_nll += r.nll;
       ++out->count;
     }
-    if (!exact)
-      for (int k = 0; k < 8; ++k) {
-        hash ^= (r.hash >> (8 * k)) & 0xFFu;
-        hash *= kFnvPrime;
-      }
+    for (int k = 0; k < 8; ++k) {
+      hash ^= (r.hash >> (8 * k)) & 0xFFu;
+      hash *= kFnvPrime;
+    }
   }
-  for (const Affine& a : ha) hash = hash * a.a + a.b;
   out->logits_hash = hash;
   return GLT_OK;
 }

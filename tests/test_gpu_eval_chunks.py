@@ -1,0 +1,33 @@
+"""Shadow-eval statistics and logits hash over every cut of the rows into
+chunks (1024 to 16 per row), rows that start off 16 bytes, and rows shorter
+than their chunks, against the oracle."""
+import numpy as np
+import pytest
+
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("B,T,V,ld", [(1, 1, 1, 1), (1, 2, 7, 9), (1, 3, 50257, 50257), (1, 5, 16392, 16400),
+                                      (2, 130, 4099, 4099), (3, 400, 515, 520), (4, 4099, 33, 33), (2, 8200, 24, 24)])
+def test_eval_stats_cuts(dev, B, T, V, ld):
+    """Hash exact; sums are f64 on both sides; nll within the f32 rounding of
+    max + log(sum exp) - label, 2^-22 of its terms per row."""
+    import torch
+    from glt_amd import ops
+    g = torch.Generator().manual_seed(B * T + V)
+    full = (torch.randn((B * T, ld), generator=g) * 3).bfloat16()
+    ids = torch.randint(0, V, (B, T), generator=g, dtype=torch.int32)
+    logits = full.cuda()[:, :V]
+    h0 = 0x9E3779B97F4A7C15
+    x = full[:, :V].float().numpy().reshape(B, T, V)
+    for h in (O.FNV_BASIS, h0):
+        r = ops.eval_stats(logits, ids.cuda(), h)
+        ref = O.eval_stats(x, ids.numpy(), h) if T > 1 else None
+        assert r["logits_hash"] == O.eval_hash_reference(x.reshape(B * T, V), h)
+        assert r["count"] == B * (T - 1)
+        assert abs(r["logits_sum"] - float(x.astype(np.float64).sum())) <= 1e-12 * float(np.abs(x).astype(np.float64).sum())
+        assert abs(r["logits_sumsq"] - float((x.astype(np.float64) ** 2).sum())) <= 1e-12 * float((x.astype(np.float64) ** 2).sum())
+        if ref:
+            assert abs(r["total_nll"] - ref["total_nll"]) <= 2.0 ** -22 * (np.log(V) + 4 * np.abs(x).max()) * B * T
