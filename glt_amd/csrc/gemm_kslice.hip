@@ -35,10 +35,12 @@ namespace glt {
 // one wavefront per SIMD pays for its loads and its MFMAs one after the other
 // (4 wavefronts of 64 x 128: loads alone 24 us, MFMAs alone 14, together 48 at
 // 512 x 4096 x 8192); the eight wavefronts here put two on each SIMD.
+//
+// ONCE loads B non-temporally (read_once below says when).
 // =========================================================================
 constexpr int min63(int n) { return n < 63 ? n : 63; }  // vmcnt holds 6 bits
 
-template <int TI, int TJ, int RB, int NWN, int NG, int PA, int PB, typename TO, int MODE, bool DUAL>
+template <int TI, int TJ, int RB, int NWN, int NG, int PA, int PB, typename TO, int MODE, bool DUAL, bool ONCE>
 __global__ void __launch_bounds__(64 * NWN * NG) gemm_kslice_kernel(const GArgs args) {
   extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
   constexpr int BM = 32 * TI, BNW = DUAL ? 16 * TJ : 32 * TJ, BN = BNW * NWN;
@@ -157,11 +159,12 @@ __global__ void __launch_bounds__(64 * NWN * NG) gemm_kslice_kernel(const GArgs 
   uint32_t sub[4];
 #pragma unroll
   for (int s = 0; s < 4; ++s) sub[s] = (s + rot) & 3;
+  constexpr int kAux = ONCE ? 2 : 0;  // 2: non-temporal
   bf16x8 fb[PB][4][TJ];
   auto load_b = [&](int u, int s, int j) {
     const __amdgpu_buffer_rsrc_t r = (DUAL && j >= TJ / 2) ? uni_rsrc(pB1, nB1) : uni_rsrc(pB0, nB0);
     const uint32_t so = (uint32_t)pb.k * 64 + sub[s] * 1024;  // 1 KB per fragment of 16 K
-    fb[u][s][j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, voB[j], so, 0));
+    fb[u][s][j] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, voB[j], so, kAux));
   };
 
   f32x16 acc[TI][TJ];
@@ -447,12 +450,12 @@ int pick_kslice(const GemmPlan& plan, int cus) {
   return best;
 }
 
-template <int TI, int TJ, int RB, int NWN, int NG, int PA, int PB, typename TO, int MODE, bool DUAL>
-static glt_status launch_ks(const GArgs& a, hipStream_t st, const char* label) {
+template <int TI, int TJ, int RB, int NWN, int NG, int PA, int PB, typename TO, int MODE, bool DUAL, bool ONCE>
+static glt_status launch_ks_as(const GArgs& a, hipStream_t st, const char* label) {
   static std::atomic<bool> attr_set[64];
   // dual tiles pair gate with up blocks (a 1 x 1 shape takes one of each)
   constexpr int TJ_ = DUAL && TJ == 1 ? 2 : TJ;
-  auto fn = gemm_kslice_kernel<TI, TJ_, RB, NWN, NG, PA, PB, TO, MODE, DUAL>;
+  auto fn = gemm_kslice_kernel<TI, TJ_, RB, NWN, NG, PA, PB, TO, MODE, DUAL, ONCE>;
   int dev = 0;
   GLT_TRY_HIP(hipGetDevice(&dev));
   GLT_CHECK(dev >= 0 && dev < 64, GLT_ERR_HIP, "gemm: device index %d out of range", dev);
@@ -467,6 +470,32 @@ static glt_status launch_ks(const GArgs& a, hipStream_t st, const char* label) {
   GLT_LAUNCH(label, fn, dim3(a.total_tiles), dim3(64 * NWN * NG), lds, st, a);
   GLT_LAUNCH_CHECK("gemm_kslice");
   return GLT_OK;
+}
+
+// Whether B is read once and gone: a single row of tiles (no other workgroup
+// reads the same part of B), and more than half of the 256 MB last-level cache
+// of it, so that the next call would not find it there whatever the loads say.
+// Non-temporal loads then stream faster and leave the cache to the others'
+// operands: MLP forward of 4096 x 15360, one layer called again and again, 8
+// tokens 81 -> 65 us, 64 tokens 91 -> 72; four layers in turn 80 -> 76 and 92
+// -> 86. Below that size repeated calls lose the cached weights (2048 x 11008,
+// 8 tokens: 34 -> 41 us), and with several row tiles the B that they share
+// comes twice (4096 x 15360, 200 tokens: 180 -> 222 us).
+static bool read_once(const GArgs& a, bool dual) {
+  int64_t bytes = 0;
+  for (int p = 0; p < a.nprob; ++p) {
+    const GProb& P = a.p[p];
+    if (P.tiles_m > 1) return false;
+    for (int i = P.seg0; i < P.seg0 + P.nseg; ++i)
+      bytes += (int64_t)std::max(0, std::min(a.s[i].n_hi, P.N) - a.s[i].n_lo) * a.s[i].K * (dual ? 4 : 2);
+  }
+  return bytes > (int64_t)128 << 20;
+}
+
+template <int TI, int TJ, int RB, int NWN, int NG, int PA, int PB, typename TO, int MODE, bool DUAL>
+static glt_status launch_ks(const GArgs& a, hipStream_t st, const char* label) {
+  return read_once(a, DUAL) ? launch_ks_as<TI, TJ, RB, NWN, NG, PA, PB, TO, MODE, DUAL, true>(a, st, label)
+                            : launch_ks_as<TI, TJ, RB, NWN, NG, PA, PB, TO, MODE, DUAL, false>(a, st, label);
 }
 
 glt_status run_kslice(GemmPlan& plan, int shape, hipStream_t st) {

@@ -30,6 +30,28 @@ def test_head_both_ways(dev, M, K, V):
         assert rel_l2(to_np(dx), (gr.double() @ w.double()).cpu().numpy()) <= 1e-6 * np.log2(V)
 
 
+@pytest.mark.parametrize("M", [1, 32, 63, 65, 128, 129])
+def test_weights_past_the_cache(dev, M):
+    """One row of tiles (up to 128 rows) over more than 128 MiB of weights,
+    which are loaded non-temporally: LM head and the dual gate/up launch."""
+    import torch
+    from glt_amd import ops
+    K, V = 4160, 16264
+    assert V * K * 2 > 128 << 20
+    g = torch.Generator(device="cuda").manual_seed(M)
+    x = torch.randn((M, K), generator=g, device="cuda").bfloat16()
+    w = torch.randn((V, K), generator=g, device="cuda").mul_(0.05).bfloat16()
+    assert_bf16_budget(to_np(ops.lm_head_fwd(x, w)), (x.double() @ w.double().t()).cpu().numpy(), q=1, what="logits")
+    wg, wu = w[:8128], w[8128:2 * 8128].contiguous()
+    wd = torch.randn((K, 8128), generator=g, device="cuda").mul_(0.05).bfloat16()
+    _, gt, up, inter = ops.mlp_forward(ops.BaseMLP(wg, wu, wd), [], x, 8128)
+    rg, ru = x.double() @ wg.double().t(), x.double() @ wu.double().t()
+    assert_bf16_budget(to_np(gt), rg.cpu().numpy(), q=1, what="gate")
+    assert_bf16_budget(to_np(up), ru.cpu().numpy(), q=1, what="up")
+    ri = torch.nn.functional.silu(rg) * ru
+    assert_bf16_budget(to_np(inter), ri.cpu().numpy(), q=3, what="inter")
+
+
 @pytest.mark.parametrize("M", [7, 40, 70, 130, 300, 520])
 def test_mlp_slices(dev, M):
     """Forward and backward with an in-place slice over base columns, one with
