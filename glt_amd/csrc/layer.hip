@@ -523,12 +523,17 @@ __global__ void __launch_bounds__(256) eval_row_stats_kernel(const uint16_t* log
 //
 // Each pass's workgroup (256 consecutive chunks) also composes its maps, and
 // the next pass's forms its chunks' starting states from them, so that between
-// two passes only one small launch runs over the workgroups. Passes 1 and 2
-// issue about 18 instructions per logit and are bound by that: with a factor
-// P^2 carried along a logit is t ^= lo, t *= P, t ^= hi, t *= P^3, two runs per
-// register as 8-bit fields 16 bits apart, which one 24-bit multiply serves (a
-// packed 16-bit multiply needs no masks: 166 against 154 us for 2048 rows of
-// 128256, where the issue of these instructions alone is 124).
+// two passes only one small launch runs over the workgroups. With a factor P^2
+// carried along a logit is t ^= lo, t *= P, t ^= hi, t *= P^3. Pass 1 needs
+// four bits of each run: a byte per run, four runs per register, P = 3 and P^3
+// = 11 mod 16 as shift-adds, 12 instructions per logit (two runs per register
+// and 24-bit multiplies, 18 instructions: 166 against 133 us for 2048 rows of
+// 128256). Pass 2 needs all eight: two runs per register as 8-bit fields 16
+// bits apart, one 24-bit multiply for both, 18 instructions (167 us, 124 of it
+// their issue; a packed 16-bit multiply needs no masks and took 12 us more in
+// each pass). Reading 525 MB takes 81 us of each pass at least. Fetching the
+// chunks' lines eight lanes to a line through LDS, or the next 128 bytes while
+// the last are walked, changed the three passes by less than 3 %.
 constexpr uint32_t kP8 = (uint32_t)(kFnvPrime & 0xFF);
 constexpr uint64_t kP2 = kFnvPrime * kFnvPrime, kP3 = kP2 * kFnvPrime;
 constexpr uint64_t inverse64(uint64_t a) {  // of an odd a, mod 2^64 (Newton, doubling the correct bits)
@@ -591,38 +596,72 @@ __global__ void __launch_bounds__(256) hash_nibble_kernel(const uint16_t* logits
   }
   Map8 f = kMapIdentity;
   if (in) {
-    // fields 0 and 16 of st[j]: runs 2 j and 2 j + 1 (times P^2; the bits
-    // above each field's 8 are left over)
-    constexpr uint32_t kFields = 0x00FF00FFu;
-    uint32_t st[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t a = HIGH ? base | (2 * j) << 4 : 2 * j, b = HIGH ? base | (2 * j + 1) << 4 : 2 * j + 1;
-      st[j] = (a | b << 16) * (uint32_t)(kP2 & 0xFF);
-    }
     int v0, v1;
     hash_chunk_range(V, shift, (int)(k & ((1 << shift) - 1)), v0, v1);
-    auto logit = [&](uint32_t lo, uint32_t hi) {  // each byte in both fields
+    const uint16_t* row = logits + (k >> shift) * ld;
+    f = 0;
+    if constexpr (!HIGH) {
+      // byte b of st[j]: run 4 j + b, its low nibble times P^2 (the byte's
+      // high nibble is left over); P = 3 and P^3 = 11 mod 16
+      constexpr uint32_t kFields = 0x0F0F0F0Fu;
+      static_assert((kFnvPrime & 15) == 3 && (kP3 & 15) == 11, "the shifts below");
+      uint32_t st[2] = {0, 0};
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i) st[i >> 2] |= (i * (uint32_t)(kP2 & 15) & 15u) << (8 * (i & 3));
+      auto logit = [&](uint32_t lo, uint32_t hi) {  // each byte in all four
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          uint32_t t = (st[j] ^ lo) & kFields;
+          t += t << 1;               // 3 t <= 45
+          t = (t ^ hi) & kFields;
+          uint32_t t3 = t + (t << 1);
+          asm("" : "+v"(t3));        // two shift-adds, not one 32-bit multiply at a quarter of their rate
+          st[j] = (t << 3) + t3;     // 11 t <= 165
+        }
+      };
+      walk_chunk(
+          row, v0, v1,
+          [&](uint32_t w) {
+            logit(__builtin_amdgcn_perm(0u, w, 0x00000000u), __builtin_amdgcn_perm(0u, w, 0x01010101u));
+          },
+          [&](uint32_t w) {
+            logit(__builtin_amdgcn_perm(0u, w, 0x00000000u), __builtin_amdgcn_perm(0u, w, 0x01010101u));
+            logit(__builtin_amdgcn_perm(0u, w, 0x02020202u), __builtin_amdgcn_perm(0u, w, 0x03030303u));
+          });
+#pragma unroll
+      for (uint32_t i = 0; i < 8; ++i)
+        f |= (((st[i >> 2] >> (8 * (i & 3))) * (uint32_t)(kP2Inv & 15)) & 15u) << (4 * i);
+    } else {
+      // fields 0 and 16 of st[j]: runs 2 j and 2 j + 1 (times P^2; the bits
+      // above each field's 8 are left over)
+      constexpr uint32_t kFields = 0x00FF00FFu;
+      uint32_t st[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        st[j] = ((st[j] ^ lo) & kFields) * kP8;
-        st[j] = ((st[j] ^ hi) & kFields) * (uint32_t)(kP3 & 0xFF);
+        const uint32_t a = base | (2 * j) << 4, b = base | (2 * j + 1) << 4;
+        st[j] = (a | b << 16) * (uint32_t)(kP2 & 0xFF);
       }
-    };
-    walk_chunk(
-        logits + (k >> shift) * ld, v0, v1,
-        [&](uint32_t w) {
-          logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
-        },
-        [&](uint32_t w) {
-          logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
-          logit(__builtin_amdgcn_perm(0u, w, 0x0C020C02u), __builtin_amdgcn_perm(0u, w, 0x0C030C03u));
-        });
-    f = 0;
+      auto logit = [&](uint32_t lo, uint32_t hi) {  // each byte in both fields
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const uint32_t s2 = ((st[j] & kFields) * (uint32_t)(kP2Inv & 0xFF)) >> (HIGH ? 4 : 0);
-      f |= ((s2 & 15u) | ((s2 >> 16) & 15u) << 4) << (8 * j);
+        for (int j = 0; j < 4; ++j) {
+          st[j] = ((st[j] ^ lo) & kFields) * kP8;
+          st[j] = ((st[j] ^ hi) & kFields) * (uint32_t)(kP3 & 0xFF);
+        }
+      };
+      walk_chunk(
+          row, v0, v1,
+          [&](uint32_t w) {
+            logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
+          },
+          [&](uint32_t w) {
+            logit(__builtin_amdgcn_perm(0u, w, 0x0C000C00u), __builtin_amdgcn_perm(0u, w, 0x0C010C01u));
+            logit(__builtin_amdgcn_perm(0u, w, 0x0C020C02u), __builtin_amdgcn_perm(0u, w, 0x0C030C03u));
+          });
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t s2 = ((st[j] & kFields) * (uint32_t)(kP2Inv & 0xFF)) >> 4;
+        f |= ((s2 & 15u) | ((s2 >> 16) & 15u) << 4) << (8 * j);
+      }
     }
     maps[k] = f;
   }
