@@ -502,7 +502,7 @@ def bench_shadow_eval(torch, F, sp, p, reps=3):
                            "frac_hbm": round(nbytes / (t_stats * 1e-3) / 1e9 / PEAK_HBM_GBPS, 4)},
             "exact_hash_ms": round(t_hash, 4),
             "eval_stats_ms": round(t_stats + t_hash, 4),
-            "hash_bound": "integer arithmetic (16 runs of the low-byte chain per logit in two passes, one 64-bit run)"}
+            "hash_bound": "integer arithmetic (eight runs of each nibble of the low byte per logit in two passes, one 64-bit run)"}
 
 
 def bench_masked_ce(torch, F, sp, p, reps=5):
