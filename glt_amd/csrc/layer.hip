@@ -921,20 +921,25 @@ struct EvalWs {
   int64_t chunks, blocks;
   int shift;
 };
+// The chunks of R rows fall where hash_shift steps down (2048 rows have 262144,
+// 2049 rows 131136), so the buffers are laid out for a bound on them that never
+// falls as rows grow: a workspace of the largest batch holds every shorter one.
+int64_t hash_chunks_bound(int64_t R) { return std::min(R << 10, std::max(R << 4, kHashThreads)); }
 EvalWs eval_ws(int64_t R) {
   EvalWs w{};
   w.shift = hash_shift(R);
   w.chunks = R << w.shift;
   w.blocks = cdiv(w.chunks, 256);
+  const int64_t chunks = hash_chunks_bound(R), blocks = cdiv(chunks, 256);
   w.rows = 0;
   w.maps_lo = up(w.rows + R * sizeof(EvalRow));
-  w.maps_hi = up(w.maps_lo + w.chunks * sizeof(Map8));
-  w.start = up(w.maps_hi + w.chunks * sizeof(Map8));
-  w.agg = up(w.start + w.chunks);
-  w.bstart_lo = up(w.agg + w.blocks * sizeof(Map8));
-  w.bstart_hi = up(w.bstart_lo + w.blocks);
-  w.aff = up(w.bstart_hi + w.blocks);
-  w.sums = up(w.aff + w.blocks * sizeof(Affine));
+  w.maps_hi = up(w.maps_lo + chunks * sizeof(Map8));
+  w.start = up(w.maps_hi + chunks * sizeof(Map8));
+  w.agg = up(w.start + chunks);
+  w.bstart_lo = up(w.agg + blocks * sizeof(Map8));
+  w.bstart_hi = up(w.bstart_lo + blocks);
+  w.aff = up(w.bstart_hi + blocks);
+  w.sums = up(w.aff + blocks * sizeof(Affine));
   w.total = up(w.sums + sizeof(EvalTotal));
   return w;
 }

@@ -532,7 +532,8 @@ glt_status glt_model_fwd(const glt_model* m, const int32_t* ids, uint16_t* logit
  * chained in row order from hash_in (one pass over the logits; a different
  * value from the reference's).
  * Synchronous; workspace: glt_eval_stats_workspace_size bytes, 256-byte
- * aligned. */
+ * aligned; the size never falls as B * T grows, so the largest batch's
+ * workspace serves every shorter one. */
 #define GLT_FNV_BASIS 1469598103934665603ULL /* the reference's offset basis, grafting.hip:505 */
 #define GLT_EVAL_HASH_REFERENCE 0
 #define GLT_EVAL_HASH_ROWS      1

@@ -105,3 +105,17 @@ def test_eval_and_graft_adamw_validation_without_gpu():
                                     ctypes.c_void_p(4096), 1 << 20, None) == 9
     assert lib.glt_adamw_graft_step(sl, 1, arr, arr, arr, None, 7, 0, 1e-4, 0.9, 0.999, 1e-8, 0.01, 1.0, None, 0,
                                     None) == 5
+
+
+def test_eval_workspace_size_never_falls_as_rows_grow():
+    """A workspace sized for the largest eval batch serves every shorter one,
+    also across the row counts at which the hash cuts rows into fewer chunks
+    (2049 rows have half the chunks of 2048)."""
+    from glt_amd import _ffi as F
+    lib = F.load()
+    last = 0
+    for rows in range(1, 40000):
+        n = lib.glt_eval_stats_workspace_size(1, rows)
+        assert n >= last, rows
+        last = n
+    assert lib.glt_eval_stats_workspace_size(4, 1025) == lib.glt_eval_stats_workspace_size(1, 4100)

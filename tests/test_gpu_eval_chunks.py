@@ -31,3 +31,29 @@ def test_eval_stats_cuts(dev, B, T, V, ld):
         assert abs(r["logits_sumsq"] - float((x.astype(np.float64) ** 2).sum())) <= 1e-12 * float((x.astype(np.float64) ** 2).sum())
         if ref:
             assert abs(r["total_nll"] - ref["total_nll"]) <= 2.0 ** -22 * (np.log(V) + 4 * np.abs(x).max()) * B * T
+
+
+def test_workspace_of_the_largest_batch(dev):
+    """One workspace, sized once for the longest batch, for shorter batches
+    whose rows are cut into more chunks: hash against the oracle, and the bytes
+    past the workspace untouched."""
+    import ctypes
+    import torch
+    from glt_amd import _ffi as F
+    lib = F.load()
+    V, largest = 40, 2052
+    n, guard = lib.glt_eval_stats_workspace_size(1, largest), 4 << 20
+    ws = torch.full((n + guard,), 0x5A, dtype=torch.uint8, device="cuda")
+    g = torch.Generator().manual_seed(V)
+    logits = (torch.randn((largest, V), generator=g) * 3).bfloat16()
+    ids = torch.randint(0, V, (largest,), generator=g, dtype=torch.int32)
+    ld, di = logits.cuda(), ids.cuda()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    for T in (largest, 2048, 1024, 257, 256, 1):
+        r = F.EvalResult()
+        assert lib.glt_eval_stats_workspace_size(1, T) <= n
+        F.call("glt_eval_stats", p(ld), V, p(di), 1, T, V, F.EVAL_HASH_REFERENCE, O.FNV_BASIS, ctypes.byref(r), p(ws), n,
+               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert r.logits_hash == O.eval_hash_reference(logits[:T].float().numpy(), O.FNV_BASIS), T
+        assert r.count == T - 1
+    assert torch.all(ws[n:] == 0x5A).item()
