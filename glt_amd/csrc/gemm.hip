@@ -1,5 +1,5 @@
 // Segment-list GEMM: the persistent gfx950 bf16 MFMA kernel, and the choice
-// between it, the K-sliced kernel and the strided one.
+// between it, the small-tile kernel and the strided one.
 #include <algorithm>
 #include <atomic>
 #include <cstdint>
@@ -739,8 +739,8 @@ glt_status run_gemm(GemmPlan& plan, hipStream_t st, bool allow_mfma) {
     int cus = 0;
     const glt_status rc = device_cus(cus);
     if (rc != GLT_OK) return rc;
-    const int shape = pick_kslice(plan, cus);
-    if (shape >= 0) return run_kslice(plan, shape, st);
+    const int shape = pick_small(plan, cus);
+    if (shape >= 0) return run_small(plan, shape, st);
   }
   if (!mfma) {
     GLT_CHECK(plan.b_kind != LD_SHUF && plan.a_kind != LD_SHUF, GLT_ERR_UNSUPPORTED,

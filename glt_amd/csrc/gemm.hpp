@@ -87,10 +87,10 @@ struct GemmPlan {
 glt_status run_gemm(GemmPlan& plan, hipStream_t st, bool allow_mfma = true);
 bool gemm_mfma_eligible(const GemmPlan& plan);
 // The MFMA kernel for launches that do not fill the chip with 256 x 256 tiles
-// (gemm_kslice.hip): the tile shape to run an MFMA-eligible plan with, or -1
+// (gemm_small.hip): the tile shape to run an MFMA-eligible plan with, or -1
 // for the persistent kernel; and the launch.
-int pick_kslice(const GemmPlan& plan, int cus);
-glt_status run_kslice(GemmPlan& plan, int shape, hipStream_t st);
+int pick_small(const GemmPlan& plan, int cus);
+glt_status run_small(GemmPlan& plan, int shape, hipStream_t st);
 // Any plan without a shuffled operand, on the strided f32-MFMA kernel.
 glt_status run_strided(GemmPlan& plan, hipStream_t st);
 // Workgroups of the persistent MFMA kernel's launch for this plan (one per 256 x 256

@@ -1,5 +1,5 @@
 // Device helpers shared by the segment-list GEMM kernels (gemm.hip,
-// gemm_kslice.hip).
+// gemm_small.hip).
 #pragma once
 
 #include "gemm.hpp"

@@ -526,7 +526,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
       int cus = 0;
       if ((s = device_cus(cus)) != GLT_OK) return s;
       // (smaller tiles leave no CU idle)
-      const int idle = pick_kslice(plan, cus) < 0 ? cus - gemm_mfma_tiles(plan) : 0;
+      const int idle = pick_small(plan, cus) < 0 ? cus - gemm_mfma_tiles(plan) : 0;
       if (idle >= 16 && (s = fork_norm_bwd(*nb, dx, d->M, d->D, idle, st, &norm_ev)) != GLT_OK) return s;
     }
     // join the helper stream even when the GEMM launch failed, so that no

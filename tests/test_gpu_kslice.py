@@ -1,6 +1,6 @@
-"""GPU parity of the K-sliced MFMA GEMM: launches of few tiles, at the edges of
+"""GPU parity of the small-tile MFMA GEMM: launches of few tiles, at the edges of
 its tile shapes (32 x 32 to 128 x 256), with reductions whose K-steps do not
-divide evenly over the wavefront groups and their unrolled steps."""
+divide evenly over the unrolled steps."""
 import numpy as np
 import pytest
 
