@@ -525,7 +525,11 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
         rmsnorm_bwd_rows_ok(dx, nb->x, nb->w, nb->dx, d->M, d->D)) {
       int cus = 0;
       if ((s = device_cus(cus)) != GLT_OK) return s;
-      // (smaller tiles leave no CU idle)
+      // Only beside the persistent kernel, one workgroup per tile and CU: small
+      // tiles get through more of them at once and share the idle CUs' caches
+      // and the memory with the norm, which is slower on a few CUs than alone on
+      // all (M = 2048, D = 1024, S = 256, 64 CUs left: call 84 -> 109 us with
+      // the fork, M = 4096, D = 2048, S = 512: 625 -> 644).
       const int idle = pick_small(plan, cus) < 0 ? cus - gemm_mfma_tiles(plan) : 0;
       if (idle >= 16 && (s = fork_norm_bwd(*nb, dx, d->M, d->D, idle, st, &norm_ev)) != GLT_OK) return s;
     }

@@ -524,6 +524,73 @@ def test_mlp_rmsnorm_bwd_in_a_graph(dev):
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("M,D,S", [(2048, 4096, 1024), (1999, 4032, 1024)])  # 504 chunks per row: ragged lanes
+def test_mlp_rmsnorm_bwd_forks_beside_the_persistent_kernel(dev, M, D, S):
+    """Weight gradients on 192 persistent tiles: the norm's backward does run on
+    the helper stream (its launch label says so), eagerly and in a graph
+    replayed three times with eager work between, with glt_mlp_bwd's and
+    glt_rmsnorm_bwd's bits every time."""
+    import ctypes
+    import torch
+    from glt_amd import _ffi as F, ops
+    I = 256
+    N = I + S
+    g = torch.Generator(device="cuda").manual_seed(M)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").mul_(0.02)
+    bf = torch.bfloat16
+    base = ops.BaseMLP(rn(I, D).to(bf), rn(I, D).to(bf), rn(D, I).to(bf))
+    gs = [ops.GraftSlice(I, S, 0, D, rn(S, D), rn(S, D), rn(S, D)).pack()]
+    x_raw, gamma, dy = rn(M, D).mul_(50).to(bf), (1 + rn(D)).to(bf), rn(M, D).mul_(50)
+    x, var = ops.rms_norm(x_raw, gamma, 1e-5)
+    _, gp, up, inter = ops.mlp_forward(base, gs, x, N)
+    dx0, g0 = ops.mlp_backward(base, gs, x, dy, N, gp, up, inter)
+    nd0 = ops.rms_norm_bwd(dx0, x_raw, gamma, var, 1e-5)
+
+    d, keep = ops._desc(base, gs, M, N, True, dy_f32=True)
+    nbytes = F.load().glt_mlp_bwd_workspace_size(ctypes.byref(d))
+    ws = torch.empty(nbytes, dtype=torch.uint8, device="cuda")
+    dx, nd = torch.empty_like(dx0), torch.empty_like(nd0)
+    grads = [torch.empty((S, D), dtype=torch.float32, device="cuda") for _ in range(3)]
+    garr = (F.GraftGrads * 1)()
+    garr[0] = F.GraftGrads(*(t.data_ptr() for t in grads))
+    b = base.c_struct()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+
+    def call():
+        F.call("glt_mlp_rmsnorm_bwd", ctypes.byref(d), ctypes.byref(b), p(x), p(dy), p(gp), p(up), p(inter), p(dx),
+               garr, p(ws), nbytes, p(x_raw), p(gamma), p(var), 1e-5,
+               p(nd), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+    def check(what):
+        torch.cuda.synchronize()
+        assert torch.equal(dx, dx0) and torch.equal(nd, nd0), what
+        for a, r in zip(grads, g0[0]):
+            assert torch.equal(a, r), what
+        for t in (dx, nd, *grads):
+            t.fill_(float("nan"))
+        torch.cuda.synchronize()
+
+    lib = F.load()
+    lib.glt_profile_enable(1)
+    call()
+    torch.cuda.synchronize()
+    labels = F.profile_collect()
+    lib.glt_profile_enable(0)
+    assert labels["rmsnorm_bwd_beside"][1] == 1 and "rmsnorm_bwd" not in labels
+    check("profiled")
+    call()
+    check("eager")
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        call()
+    for rep in range(3):
+        graph.replay()
+        check(rep)
+        _ = (x_raw.float() * 2).sum()   # eager work between replays
+
+
 def test_outputs_past_two_gib_split_into_row_blocks(dev):
     """65536 tokens at N = 16384: the gate/up outputs and the dInter GEMM's
     outputs and saved pre-activations pass 2 GiB, beyond the MFMA kernel's
