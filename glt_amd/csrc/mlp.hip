@@ -175,6 +175,17 @@ static bool wgrad_uses_mfma(const glt_mlp_desc* d) {
   return (rows + 256) * wgrad_k(d) * 2 < (int64_t)kOob;
 }
 
+// Whether the buffers that the weight gradients alone read and write start where
+// the MFMA path needs them (inter only where its transpose is padded: whole
+// 64-token tiles have a scalar form); any other alignment runs strided.
+static bool wgrad_aligned(const glt_mlp_desc* d, const void* inter, const glt_graft_grads* grads) {
+  uintptr_t bits = d->M % 64 ? reinterpret_cast<uintptr_t>(inter) : 0;
+  for (int j = 0; j < d->n_slices; ++j)
+    bits |= reinterpret_cast<uintptr_t>(grads[j].gate) | reinterpret_cast<uintptr_t>(grads[j].up) |
+            reinterpret_cast<uintptr_t>(grads[j].down);
+  return bits % 16 == 0;
+}
+
 static BwdLayout bwd_layout(const glt_mlp_desc* d) {
   BwdLayout L{};
   const size_t es = esize(d->dtype);
@@ -358,6 +369,8 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
   void* du = W + L.du;
 
   const bool grads_wanted = explicit_graft && d->n_slices > 0;
+  const bool wgrad_mfma =
+      grads_wanted && L.wgrad_mfma && wgrad_aligned(d, recompute ? W + L.inter : inter, grads);
   bool operands_laid_out = false;  // x and dy already in the weight-gradient fragment layout
   if (L.dy_f32) {
     // The reference multiplies its f32 upstream gradient by the f32 copy of
@@ -370,7 +383,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
     const float* dyf = static_cast<const float*>(dy);
     uint16_t* XS = reinterpret_cast<uint16_t*>(W + L.xt);
     uint16_t* DYS = reinterpret_cast<uint16_t*>(W + L.dyt);
-    if (L.wgrad_mfma && grads_wanted && shuffle_tr_pair_f32_ok(x, dyf, d->D, d->D, d->M, XS, DYS, dyb)) {
+    if (wgrad_mfma && shuffle_tr_pair_f32_ok(x, dyf, d->D, d->D, d->M, XS, DYS, dyb)) {
       if ((s = shuffle_tr_pair_f32(static_cast<const uint16_t*>(x), dyf, d->D, d->D, d->M, XS, DYS, dyb, st)) !=
           GLT_OK)
         return s;
@@ -458,7 +471,7 @@ static glt_status mlp_bwd_impl(const glt_mlp_desc* d, const glt_base_weights* w,
   //    (reference src/graft_ops_impl.inc:120-141, :214-228):
   //      dGate = dgate_i^T . x_h, dUp = dup_i^T . x_h, dDown = inter_i^T . dy_h
   if (!explicit_graft || d->n_slices == 0) return GLT_OK;
-  if (L.wgrad_mfma) {
+  if (wgrad_mfma) {
     // K (= tokens) must be the contiguous axis of A: each slice's column
     // block of dgate/dup/inter is transposed once; x and dy become shuffled
     // B operands [D rows, K = M] once for all slices.

@@ -125,6 +125,52 @@ def test_ragged_weight_gradients(dev, M):
             assert torch.equal(grads[j][p], grads32[j][p])
 
 
+@pytest.mark.parametrize("M", [65, 128])
+@pytest.mark.parametrize("what", ["gate", "up", "down", "inter"])
+@pytest.mark.parametrize("recompute", [False, True])
+def test_weight_gradients_off_16_bytes(dev, M, what, recompute):
+    """A gradient buffer 4 bytes, or the saved inter 2, past a 16-byte boundary:
+    the same bf16 operands, read by the strided kernel or its scalar transpose.
+    f32 sums of exact products: rel-L2 within 1e-6 per doubling of the number of terms, and
+    nothing written around the buffer."""
+    import ctypes
+    import torch
+    from glt_amd import _ffi as F, ops
+    if what == "inter" and recompute:
+        pytest.skip("inter is recomputed into the workspace")
+    D, I, S, H0, H = 512, 1024, 128, 64, 384
+    N = I + S
+    g = torch.Generator(device="cuda").manual_seed(M)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").mul_(0.02)
+    bf = torch.bfloat16
+    base = ops.BaseMLP(rn(I, D).to(bf), rn(I, D).to(bf), rn(D, I).to(bf))
+    gs = [ops.GraftSlice(I, S, H0, H, rn(S, H), rn(S, H), rn(S, H)).pack()]
+    x, dy = rn(M, D).mul_(50).to(bf), rn(M, D).mul_(50).to(bf)
+    _, gp, up, inter = ops.mlp_forward(base, gs, x, N)
+    dx0, g0 = ops.mlp_backward(base, gs, x, dy, N, gp, up, inter)
+
+    d, keep = ops._desc(base, gs, M, N, True, recompute=recompute)
+    n = F.load().glt_mlp_bwd_workspace_size(ctypes.byref(d))
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    store = [torch.full((S * H + 8,), 7.0, device="cuda") for _ in range(3)]
+    off = [1 if name == what else 0 for name in ("gate", "up", "down")]
+    garr = (F.GraftGrads * 1)()
+    garr[0] = F.GraftGrads(*(t.data_ptr() + 4 * o for t, o in zip(store, off)))
+    if what == "inter":
+        odd = torch.empty(M * N + 1, dtype=bf, device="cuda")
+        odd[1:] = inter.reshape(-1)
+        inter = odd[1:]
+    dx = torch.empty_like(dx0)
+    b = base.c_struct()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    F.call("glt_mlp_bwd", ctypes.byref(d), ctypes.byref(b), p(x), p(dy), p(gp), p(up), p(inter), p(dx), garr, p(ws), n,
+           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert torch.equal(dx, dx0)
+    for t, o, ref in zip(store, off, g0[0]):
+        assert rel_l2(to_np(t[o:o + S * H]), to_np(ref).reshape(-1)) <= 1e-6 * np.log2(M)
+        assert torch.all(t[:o] == 7.0) and torch.all(t[o + S * H:] == 7.0)
+
+
 def _graft_rows(gs, dy, N):
     import torch
     out = torch.zeros((dy.shape[0], N), device="cuda")
