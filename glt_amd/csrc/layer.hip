@@ -408,13 +408,14 @@ __global__ void __launch_bounds__(256) eval_row_stats_kernel(const uint16_t* log
   const int64_t r = blockIdx.x;
   const uint16_t* x = logits + r * ld;
   double s = 0.0, s2 = 0.0;
-  // The running maximum starts finite and low (-2^126: times log2(e) it
-  // stays finite), so exp(-inf - m) is 0 and the first chunk's rescale of
-  // the zero sum needs no test. Each chunk rescales the sum to the new
-  // maximum (a factor of 1 when it did not grow), branch-free; exp(x - m)
-  // is exp2(x log2(e) - m log2(e)), one fma per logit.
+  // The running maximum starts at the lowest finite value, so exp(-inf - m) is
+  // 0 and the first chunk's rescale of the zero sum needs no test. Each chunk
+  // rescales the sum to the new maximum (a factor of 1 when it did not grow),
+  // branch-free; exp(x - m) is exp2((x - m) log2(e)): x log2(e) - m log2(e) in one
+  // fma, as fast (the pass waits for memory), is off by the rounding of m log2(e),
+  // which past m = 1e9 is more than exp2's range.
   constexpr float kLog2e = 1.4426950408889634f;
-  float m = -8.5070592e37f, se = 0.f;
+  float m = -3.4028235e38f, se = 0.f;
   auto add8 = [&](const u32x4& q) {
     float f[8];
 #pragma unroll
@@ -426,12 +427,11 @@ __global__ void __launch_bounds__(256) eval_row_stats_kernel(const uint16_t* log
 #pragma unroll
     for (int e = 1; e < 8; ++e) lm = fmaxf(lm, f[e]);
     const float mn = fmaxf(m, lm);
-    const float mn2 = mn * kLog2e;
-    se *= __builtin_amdgcn_exp2f(fmaf(m, kLog2e, -mn2));
+    se *= __builtin_amdgcn_exp2f((m - mn) * kLog2e);
     m = mn;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-      se += __builtin_amdgcn_exp2f(fmaf(f[e], kLog2e, -mn2));
+      se += __builtin_amdgcn_exp2f((f[e] - mn) * kLog2e);
       // squared in f64 like the reference (static_cast<double>(f) * f): the
       // f32 square of a large or tiny logit overflows or underflows; the
       // product of two f32 values is exact in f64, so one fma is the

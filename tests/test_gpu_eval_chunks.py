@@ -33,6 +33,46 @@ def test_eval_stats_cuts(dev, B, T, V, ld):
             assert abs(r["total_nll"] - ref["total_nll"]) <= 2.0 ** -22 * (np.log(V) + 4 * np.abs(x).max()) * B * T
 
 
+@pytest.mark.parametrize("V", [33, 32, 4099, 4096])
+def test_logits_at_the_ends_of_the_range(dev, V):
+    """Rows that hold the type's largest value, only its lowest, a mask of the
+    lowest and of -inf beside ordinary logits, and rows of infinities: nll as
+    max + log(sum exp(x - max)) - label gives it in f64, within f32 rounding of
+    its terms, NaN where that is NaN."""
+    import torch
+    from glt_amd import ops
+    big = torch.finfo(torch.bfloat16).max
+    g = torch.Generator().manual_seed(V)
+    base = (torch.randn((2, V), generator=g) * 3).bfloat16()
+    rows = []
+    for kind in range(8):
+        r = base.clone()
+        if kind == 0: r[0, V // 2] = big
+        if kind == 1: r[0] = -big
+        if kind == 2: r[0, ::2] = -big
+        if kind == 3: r[0, 1::2] = -float("inf")
+        if kind == 4: r[0, 1:] = -float("inf")
+        if kind == 5: r[0] = -float("inf")
+        if kind == 6: r[0, V - 1] = float("inf")
+        if kind == 7: r[0] = torch.where(r[0] > 0, 1.5e38, -1.5e38)
+        rows.append(r)
+    for kind, r in enumerate(rows):
+        for label in (0, V - 2):
+            ids = torch.tensor([[0, label]], dtype=torch.int32)
+            got = ops.eval_stats(r.cuda(), ids.cuda())
+            z = r[0].double()
+            m = z.max()
+            want = (m + torch.log(torch.exp(z - m).sum()) - z[label]).item()
+            nll = got["total_nll"]
+            if want != want:
+                assert nll != nll, (kind, label, nll)
+            elif abs(want) == float("inf"):
+                assert nll == want, (kind, label, nll)
+            else:
+                terms = abs(m.item()) + abs(z[label].item()) + np.log(V)
+                assert abs(nll - want) <= 2.0 ** -22 * terms, (kind, label, nll, want)
+
+
 def test_workspace_of_the_largest_batch(dev):
     """One workspace, sized once for the longest batch, for shorter batches
     whose rows are cut into more chunks: hash against the oracle, and the bytes
