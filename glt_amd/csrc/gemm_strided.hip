@@ -1,5 +1,6 @@
 // Segment-list GEMM over strided operands: the f32 path, bf16 shapes that the
 // fragment layout does not take, and the graft-GEMM probes.
+#include <algorithm>
 #include <atomic>
 
 #include "gemm.hpp"
@@ -92,7 +93,9 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int tm, tn;
-  const int pi = locate_tile(args, blockIdx.x, tm, tn);
+  const int64_t t = (int64_t)blockIdx.y * gridDim.x + blockIdx.x;
+  if (t >= args.total_tiles) return;
+  const int pi = locate_tile(args, (int)t, tm, tn);
   const GProb& P = args.p[pi];
   const int m0 = tm * TILE, n0 = tn * TILE, send = P.seg0 + P.nseg;
 
@@ -258,7 +261,11 @@ static glt_status launch_strided(GemmPlan& plan, hipStream_t st) {
   }
   a.total_tiles = (int)tiles;
   if (tiles == 0) return GLT_OK;
-  GLT_LAUNCH(plan.label, fn, dim3(a.total_tiles), dim3(64 * NW), lds, st, a);
+  // (a grid dimension holds at most 2^32 threads: 2^24 tiles of 256, e.g. 2^29
+  // rows of a 1-column layer)
+  constexpr int64_t kGridX = 1 << 20;
+  const dim3 grid((unsigned)std::min(tiles, kGridX), (unsigned)cdiv(tiles, kGridX));
+  GLT_LAUNCH(plan.label, fn, grid, dim3(64 * NW), lds, st, a);
   GLT_LAUNCH_CHECK("gemm_strided");
   return GLT_OK;
 }

@@ -62,3 +62,20 @@ def test_f32_mlp(dev, M, D, I, pl):
     for j in range(len(pl)):
         for p in range(3):
             assert rel_l2(to_np(grads[j][p]), rgr[j][p]) <= 1e-5, (j, p)
+
+
+def test_more_tiles_than_a_grid_dimension_holds(dev):
+    """A gate/up launch of 2^24 + 2 tiles (2^29 + 64 rows of one column): y of
+    every row, x holding one of four values."""
+    import torch
+    from glt_amd import ops
+    M = (1 << 29) + 64
+    one = torch.full((1, 1), 1.0, device="cuda")
+    base = ops.BaseMLP(one, one, one)
+    vals = torch.tensor([-2.0, 0.5, 1.0, 3.0], device="cuda")
+    x = vals.repeat(M // 4).view(M, 1)
+    y, _, _, inter = ops.mlp_forward(base, [], x, 1, save=False)
+    ref, _, _, _ = ops.mlp_forward(base, [], vals.view(4, 1).contiguous(), 1, save=False)
+    assert torch.equal(y.view(M // 4, 4), ref.view(1, 4).expand(M // 4, 4))
+    want = torch.nn.functional.silu(vals.double()) * vals.double()
+    assert rel_l2(to_np(ref.view(-1)), want.cpu().numpy()) <= 1e-6
