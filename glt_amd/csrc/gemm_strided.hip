@@ -100,7 +100,8 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   const int m0 = tm * TILE, n0 = tn * TILE, send = P.seg0 + P.nseg;
 
   // ---- chunk position: segment s, offset k0 in it
-  int s = P.seg0 - 1, k0 = 0, K = 0;
+  int s = P.seg0 - 1;
+  uint32_t k0 = 0, K = 0;
   // Four-element pieces of one operand's chunk: piece q of a thread is number e
   // = tid + 64 NW q. Along k: a wavefront takes PR rows x PK pieces (256 bytes
   // of a row, and transposing writes that cover all banks). Along the rows:
@@ -109,17 +110,17 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   constexpr int PK = BK / 4 < 16 ? BK / 4 : 16, PR = 64 / PK;
   struct Src {
     const char* p[2];  // piece q of the chunk at k0
-    int k[2];          // its k within a chunk, or past any K for a row outside the operand
+    uint32_t k[2];     // its k within a chunk, or past any K for a row outside the operand
     int off[2], inc;   // where its elements go in the staged [k][row] tile
     int mode;
     int64_t step, ks;  // bytes per chunk, per k
   };
-  constexpr int kNoRow = 1 << 30;
+  constexpr uint32_t kNoRow = 0x80000000u;  // (k0 + kNoRow + 3 stays in 32 bits: k0 is a multiple of 16 below 2^31)
   Src sa, sb[NB];
   f32x4 ra[2], rb[NB][2];
   auto setup = [&](auto kind, Src& r, const StridedOp& o, int base) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind)::value, E = KIND == LD_BF16 ? 2 : 4;
-    r.mode = o.p ? piece_mode<KIND>(o, K) : PIECE_NONE;
+    r.mode = o.p ? piece_mode<KIND>(o, (int)K) : PIECE_NONE;
     r.ks = o.ks * E;
     r.step = r.ks * BK;
     r.inc = r.mode == PIECE_ROW ? 1 : PITCH;
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
       const int row = r.mode == PIECE_ROW ? 4 * (e % (TILE / 4)) : e / PK % PR + PR * (e / 64 / (BK / 4 / PK));
       const int k = r.mode == PIECE_ROW ? e / (TILE / 4) : 4 * (e % PK + PK * (e / 64 % (BK / 4 / PK)));
       const bool in = o.p && base + row >= o.lo && base + row < o.hi;
-      r.k[q] = in ? k : kNoRow;
+      r.k[q] = in ? (uint32_t)k : kNoRow;
       r.off[q] = k * PITCH + row;
       r.p[q] = static_cast<const char*>(o.p) + ((int64_t)(base + row - o.r0) * o.ld + (int64_t)k * o.ks) * E;
     }
@@ -161,7 +162,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
     k0 = 0;
     if (s >= send) return;
     const GSeg& S = args.s[s];
-    K = S.K;
+    K = (uint32_t)S.K;
     const int64_t ae = LA == LD_BF16 ? 2 : 4;
     setup(Kind<LA>{}, sa,
           StridedOp{static_cast<const char*>(S.A) + (int64_t)S.a_col * S.a_ks * ae, S.lda, S.a_ks, 0, 0, P.M}, m0);

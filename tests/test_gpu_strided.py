@@ -79,3 +79,20 @@ def test_more_tiles_than_a_grid_dimension_holds(dev):
     assert torch.equal(y.view(M // 4, 4), ref.view(1, 4).expand(M // 4, 4))
     want = torch.nn.functional.silu(vals.double()) * vals.double()
     assert rel_l2(to_np(ref.view(-1)), want.cpu().numpy()) <= 1e-6
+
+
+def test_reductions_past_two_to_the_thirty(dev):
+    """One output over more than 2^30 terms: zeros but for a few terms at both
+    ends and in the middle, summed exactly."""
+    import torch
+    from glt_amd import _ffi as F, ops
+    H = (1 << 30) + 44
+    a = torch.zeros((1, H), dtype=torch.bfloat16, device="cuda")
+    delta = torch.zeros((1, H), device="cuda")
+    want = 0.0
+    for k, t in enumerate((0, 1, 255, 256, H // 2, (1 << 30) - 1, 1 << 30, H - 2, H - 1)):
+        a[0, t], delta[0, t] = k + 1, 2.0 ** k
+        want += (k + 1) * 2.0 ** k
+    out = torch.empty((1, 1), device="cuda")
+    ops.graft_gemm(F.GEMM_EXPAND_FWD, 1, 1, H, out, a=a, lda=H, delta=delta)
+    assert out.item() == want
