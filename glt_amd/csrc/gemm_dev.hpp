@@ -45,9 +45,21 @@ __device__ __forceinline__ float round_like(float v) {
   else return bf16_to_f32(bf16_hw(v));
 }
 
+// The saved pre-activations that the EPI_DGDU form of epilogue() reads.
+struct SavedGU {
+  float g, u;
+};
+template <typename TO, int MODE>
+__device__ __forceinline__ SavedGU load_saved(const GProb& P, int m, int n) {
+  if constexpr (MODE != EPI_DGDU) return SavedGU{};
+  if (m >= P.M || n >= P.N) return SavedGU{};
+  const int64_t oa = (int64_t)m * P.ldaux + n;
+  return SavedGU{ld_elem<TO>(P.aux0, oa), ld_elem<TO>(P.aux1, oa)};
+}
+
 // a0 = accumulator (gate accumulator in the dual form), a1 = up accumulator.
 template <typename TO, int MODE>
-__device__ __forceinline__ void epilogue(const GProb& P, int m, int n, float a0, float a1) {
+__device__ __forceinline__ void epilogue(const GProb& P, int m, int n, float a0, float a1, SavedGU saved) {
   if (m >= P.M || n >= P.N) return;
   const int64_t o = (int64_t)m * P.ldo + n;
   if constexpr (MODE == EPI_STORE) {
@@ -72,8 +84,7 @@ __device__ __forceinline__ void epilogue(const GProb& P, int m, int n, float a0,
   } else {
     // SiLU*up derivative on the dInter accumulator
     // (reference fused_gate_up_bwd_kernel, src/kernels_elementwise_impl.inc:107-117).
-    const int64_t oa = (int64_t)m * P.ldaux + n;
-    const float g = ld_elem<TO>(P.aux0, oa), u = ld_elem<TO>(P.aux1, oa);
+    const float g = saved.g, u = saved.u;
     const float sg = sigmoid_fast(g);
     const float gv = g * sg;
     const float sgrad = sg * (1.0f + g * (1.0f - sg));

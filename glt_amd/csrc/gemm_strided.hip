@@ -59,37 +59,50 @@ __device__ __forceinline__ int piece_mode(const StridedOp& o, int K) {
 // f32 MFMA kernel (v_mfma_f32_32x32x2_f32: f32 products, f32 sums), operands
 // of any stride converted to f32 as they are staged.
 //
+// Every output is the sum, in order, of 16 partial sums (dual: 8); part p takes
+// the groups of 16 K whose number in their segment is p mod 16, each from its
+// segments' first group to the last. So a row's bits depend neither on the rows
+// beside it nor on which of the forms below a launch of that size takes.
+//
 // TILE 32: one 32 x 32 output tile per workgroup of NW wavefronts (dual: the
 // gate and up columns of it); each wavefront takes 16 K of every chunk of 16
-// NW, and the NW partial tiles are added through LDS at the end. A chunk costs
-// a load latency whatever its size, so launches of few tiles take many
-// wavefronts (M = N = 512, K = 3328: 98 us with 4). TILE 64: one 64 x 64 tile,
-// a 32 x 32 quadrant per wavefront over chunks of 32 K: half the operand bytes
-// per product, for launches that fill the chip with those.
+// NW, into its accumulators (one per part) in turn. A chunk costs a load latency
+// whatever its size, so launches of few tiles take many wavefronts (M = N = 512,
+// K = 3328: 33 us with 16, 98 with 4). TILE 64: one 64 x 64 tile, a 32 x 32
+// quadrant per four wavefronts over chunks of 64 K, 16 each: half the operand
+// bytes per product, for launches that fill the chip with those.
 //
 // Operand tiles are staged as [k][row] in two LDS buffers (a row of 32 or 64
 // floats plus one: the transposing writes of four k and the reads of 32 rows
 // both spread over the banks); the next chunk's global loads are in flight
 // during the MFMAs of the current one. Bound by the f32 MFMA rate (64 cycles
 // per 4096 FLOP and SIMD) once the loads are 16 bytes wide: the 512-token f32
-// layer's GEMMs took 1286 us on the FMA kernel with scalar loads this
-// replaced.
+// layer's GEMMs (hidden 512, base 1408, slice 256) take 125 us, 1286 on an FMA
+// kernel with scalar loads. The accumulators of the parts cost little against
+// one each (2048 tokens of 1024 x 2816: 1148 us and 1117; dInter 203 and 171,
+// its 16-wavefront tiles share no CU) and halve the distance to 64-bit sums
+// (6.6e-7 -> 4.1e-7). The dual form of four wavefronts is held to three a SIMD:
+// left to itself the compiler takes registers for two (329 -> 383 us).
 // =========================================================================
 template <bool DUAL, int TILE, int NW>
 struct StridedGeom {
-  static constexpr int BK = TILE == 32 ? 16 * NW : 32, NB = DUAL ? 2 : 1, PITCH = TILE + 1;
+  static constexpr int kParts = DUAL ? 8 : 16;
+  static constexpr int BK = TILE == 32 ? 16 * NW : 64, NB = DUAL ? 2 : 1, PITCH = TILE + 1;
   static constexpr int kOp = BK * PITCH;           // floats of one staged operand
   static constexpr int kStage = (1 + NB) * kOp;    // one buffer
-  static constexpr int kLds = 2 * kStage * 4;
-  static_assert(TILE == 32 || (TILE == 64 && NW == 4 && !DUAL), "64 x 64 tiles: four quadrants");
-  static_assert(TILE == 64 || kLds >= NB * NW * 32 * 33 * 4, "the partial tiles fit the buffers");
+  static constexpr int kRed = NB * NW * 32 * 33;   // floats of one partial tile of every wavefront
+  static constexpr int kLds = (2 * kStage > kRed ? 2 * kStage : kRed) * 4;
+  static constexpr int kAcc = kParts * 16 / BK;                       // accumulators of a wavefront
+  static constexpr int kPieces = BK * TILE / (4 * 64 * NW);           // 4-element pieces of a thread and operand
+  static_assert(TILE == 32 || (TILE == 64 && NW == 16 && !DUAL), "64 x 64 tiles: four quadrants, four wavefronts each");
   static_assert(kLds <= 160 * 1024, "LDS of one CU");
 };
 
 template <int LA, int LB, typename TO, int MODE, bool DUAL, int TILE, int NW>
-__global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args) {
+__global__ void __launch_bounds__(64 * NW, DUAL && NW == 4 ? 3 : 1) gemm_strided_kernel(const GArgs args) {
   using Geom = StridedGeom<DUAL, TILE, NW>;
   constexpr int BK = Geom::BK, NB = Geom::NB, PITCH = Geom::PITCH, kOp = Geom::kOp, kThreads = 64 * NW;
+  constexpr int NACC = Geom::kAcc, NQ = Geom::kPieces;
   extern __shared__ __attribute__((aligned(16))) float lds[];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   int tm, tn;
@@ -109,15 +122,15 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   // (formed per chunk they were half of the loop's instructions).
   constexpr int PK = BK / 4 < 16 ? BK / 4 : 16, PR = 64 / PK;
   struct Src {
-    const char* p[2];  // piece q of the chunk at k0
-    uint32_t k[2];     // its k within a chunk, or past any K for a row outside the operand
-    int off[2], inc;   // where its elements go in the staged [k][row] tile
+    const char* p[NQ];  // piece q of the chunk at k0
+    uint32_t k[NQ];    // its k within a chunk, or past any K for a row outside the operand
+    int off[NQ], inc;  // where its elements go in the staged [k][row] tile
     int mode;
     int64_t step, ks;  // bytes per chunk, per k
   };
   constexpr uint32_t kNoRow = 0x80000000u;  // (k0 + kNoRow + 3 stays in 32 bits: k0 is a multiple of 16 below 2^31)
   Src sa, sb[NB];
-  f32x4 ra[2], rb[NB][2];
+  f32x4 ra[NQ], rb[NB][NQ];
   auto setup = [&](auto kind, Src& r, const StridedOp& o, int base) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind)::value, E = KIND == LD_BF16 ? 2 : 4;
     r.mode = o.p ? piece_mode<KIND>(o, (int)K) : PIECE_NONE;
@@ -125,7 +138,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
     r.step = r.ks * BK;
     r.inc = r.mode == PIECE_ROW ? 1 : PITCH;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < NQ; ++q) {
       const int e = tid + kThreads * q;
       const int row = r.mode == PIECE_ROW ? 4 * (e % (TILE / 4)) : e / PK % PR + PR * (e / 64 / (BK / 4 / PK));
       const int k = r.mode == PIECE_ROW ? e / (TILE / 4) : 4 * (e % PK + PK * (e / 64 % (BK / 4 / PK)));
@@ -138,7 +151,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   auto fetch = [&](auto kind, Src& o, f32x4* r) __attribute__((always_inline)) {
     constexpr int KIND = decltype(kind)::value;
 #pragma unroll
-    for (int q = 0; q < 2; ++q) {
+    for (int q = 0; q < NQ; ++q) {
       r[q] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (o.mode != PIECE_NONE) {
         if (k0 + o.k[q] < K) r[q] = ld4_kind<KIND>(o.p[q], 0);
@@ -152,7 +165,7 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
   };
   auto put = [&](float* dst, const Src& o, const f32x4* r) __attribute__((always_inline)) {
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < NQ; ++q)
 #pragma unroll
       for (int i = 0; i < 4; ++i) dst[o.off[q] + i * o.inc] = r[q][i];
   };
@@ -179,61 +192,81 @@ __global__ void __launch_bounds__(64 * NW) gemm_strided_kernel(const GArgs args)
     for (int h = 0; h < NB; ++h) fetch(Kind<LB>{}, sb[h], rb[h]);
   };
 
-  f32x16 acc[NB];
+  f32x16 acc[NB][NACC];
 #pragma unroll
-  for (int h = 0; h < NB; ++h) acc[h] = f32x16{};
+  for (int h = 0; h < NB; ++h)
+#pragma unroll
+    for (int j = 0; j < NACC; ++j) acc[h][j] = f32x16{};
   const int lr = lane & 31, lk = lane >> 5;
-  const int kw = TILE == 32 ? 16 * wave : 0;                                  // this wavefront's first k of a chunk
-  const int am = TILE == 32 ? 0 : 32 * (wave >> 1), bn = TILE == 32 ? 0 : 32 * (wave & 1);
+  // this wavefront's first k of a chunk, rows and columns of the tile
+  const int kw = 16 * (TILE == 32 ? wave : wave >> 2);
+  const int am = TILE == 32 ? 0 : 32 * (wave >> 1 & 1), bn = TILE == 32 ? 0 : 32 * (wave & 1);
   next_seg();
   if (s < send) load();
   int p = 0;
   while (s < send) {
-    float* const st = lds + p * Geom::kStage;
-    p ^= 1;
-    put(st, sa, ra);
+    // the chunks of one turn through the accumulators, or those left of the segment
 #pragma unroll
-    for (int h = 0; h < NB; ++h) put(st + (1 + h) * kOp, sb[h], rb[h]);
-    k0 += BK;
-    if (k0 >= K) next_seg();
-    __syncthreads();  // (whoever writes the other buffer next has passed this barrier after reading it)
-    if (s < send) load();
+    for (int j = 0; j < NACC; ++j) {
+      float* const st = lds + p * Geom::kStage;
+      p ^= 1;
+      put(st, sa, ra);
 #pragma unroll
-    for (int k = 0; k < (TILE == 32 ? 16 : 32); k += 2) {
-      const int o = (kw + k + lk) * PITCH + lr;
-      const float a = st[o + am];
+      for (int h = 0; h < NB; ++h) put(st + (1 + h) * kOp, sb[h], rb[h]);
+      k0 += BK;
+      const bool last = k0 >= K;
+      if (last) next_seg();
+      __syncthreads();  // (whoever writes the other buffer next has passed this barrier after reading it)
+      if (s < send) load();
 #pragma unroll
-      for (int h = 0; h < NB; ++h)
-        acc[h] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[(1 + h) * kOp + o + bn], acc[h], 0, 0, 0);
+      for (int k = 0; k < 16; k += 2) {
+        const int o = (kw + k + lk) * PITCH + lr;
+        const float a = st[o + am];
+#pragma unroll
+        for (int h = 0; h < NB; ++h)
+          acc[h][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a, st[(1 + h) * kOp + o + bn], acc[h][j], 0, 0, 0);
+      }
+      if (last) break;
     }
   }
 
-  // lane l holds output column l & 31, rows 8 (e >> 2) + 4 (l >> 5) + (e & 3)
-  if constexpr (TILE == 64) {
+  // The parts are added through LDS, an accumulator of every wavefront at a
+  // time: lane l holds output column l & 31, rows 8 (e >> 2) + 4 (l >> 5) + (e &
+  // 3); [operand][wavefront][32 rows][33].
+  constexpr int NV = TILE * TILE / kThreads;  // a thread's outputs
+  float v[NV][2];
+  SavedGU saved[NV];  // in flight meanwhile
 #pragma unroll
-    for (int e = 0; e < 16; ++e)
-      epilogue<TO, MODE>(P, m0 + am + 8 * (e >> 2) + 4 * lk + (e & 3), n0 + bn + lr, acc[0][e], 0.f);
-  } else {
-    float* const red = lds;  // [operand][wavefront][32 rows][33]
+  for (int i = 0; i < NV; ++i) {
+    const int e = tid + kThreads * i;
+    v[i][0] = v[i][1] = 0.f;
+    saved[i] = load_saved<TO, MODE>(P, m0 + e / TILE, n0 + e % TILE);
+  }
+#pragma unroll
+  for (int j = 0; j < NACC; ++j) {
     __syncthreads();
 #pragma unroll
     for (int h = 0; h < NB; ++h)
 #pragma unroll
       for (int e = 0; e < 16; ++e)
-        red[((h * NW + wave) * 32 + 8 * (e >> 2) + 4 * lk + (e & 3)) * 33 + lr] = acc[h][e];
+        lds[((h * NW + wave) * 32 + 8 * (e >> 2) + 4 * lk + (e & 3)) * 33 + lr] = acc[h][j][e];
     __syncthreads();
 #pragma unroll
-    for (int e = tid; e < 32 * 32; e += kThreads) {
-      const int row = e >> 5, col = e & 31;
-      float v[2] = {0.f, 0.f};
+    for (int i = 0; i < NV; ++i) {
+      const int e = tid + kThreads * i, row = e / TILE, col = e % TILE;
 #pragma unroll
-      for (int h = 0; h < NB; ++h) {
-        const float* r = red + (h * NW * 32 + row) * 33 + col;
+      for (int h = 0; h < NB; ++h)
 #pragma unroll
-        for (int w = 0; w < NW; ++w) v[h] += r[w * 32 * 33];
-      }
-      epilogue<TO, MODE>(P, m0 + row, n0 + col, v[0], v[1]);
+        for (int w = 0; w < (TILE == 32 ? NW : 4); ++w) {
+          const int from = TILE == 32 ? w : 4 * w + 2 * (row >> 5) + (col >> 5);
+          v[i][h] += lds[((h * NW + from) * 32 + (row & 31)) * 33 + (col & 31)];
+        }
     }
+  }
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int e = tid + kThreads * i;
+    epilogue<TO, MODE>(P, m0 + e / TILE, n0 + e % TILE, v[i][0], v[i][1], saved[i]);
   }
 }
 
@@ -284,15 +317,15 @@ glt_status run_strided(GemmPlan& plan, hipStream_t st) {
   int cus = 0;
   const glt_status rc = device_cus(cus);
   if (rc != GLT_OK) return rc;
-  // 64 x 64 tiles where there are several per CU, else 32 x 32 with the more
-  // wavefronts the fewer tiles there are
-  const bool big = tiles64 >= 3 * (int64_t)cus, few = tiles32 <= cus, some = tiles32 <= (plan.dual ? 1 : 2) * (int64_t)cus;
+  // 64 x 64 tiles where there are several per CU, else 32 x 32, with the more
+  // wavefronts where there is less than one per CU
+  const bool big = tiles64 >= 3 * (int64_t)cus, few = tiles32 <= cus;
 #define GLT_STRIDED(LA_, LB_, TO_, MODE_, DUAL_)                                                          \
   if (la == LA_ && lb == LB_ && (sizeof(TO_) == 4) == (of32 != 0) && mode == MODE_ && plan.dual == DUAL_) \
-    return big && !DUAL_   ? launch_strided<LA_, LB_, TO_, MODE_, DUAL_, DUAL_ ? 32 : 64, 4>(plan, st)    \
+    return big && !DUAL_   ? launch_strided<LA_, LB_, TO_, MODE_, DUAL_, DUAL_ ? 32 : 64, DUAL_ ? 8 : 16>(plan, st)    \
            : few && !DUAL_ ? launch_strided<LA_, LB_, TO_, MODE_, DUAL_, 32, DUAL_ ? 8 : 16>(plan, st)    \
-           : some          ? launch_strided<LA_, LB_, TO_, MODE_, DUAL_, 32, 8>(plan, st)                 \
-                           : launch_strided<LA_, LB_, TO_, MODE_, DUAL_, 32, 4>(plan, st);
+           : few || !DUAL_ ? launch_strided<LA_, LB_, TO_, MODE_, DUAL_, 32, 8>(plan, st)                 \
+                           : launch_strided<LA_, LB_, TO_, MODE_, DUAL_, 32, DUAL_ ? 4 : 8>(plan, st);
   // f32 path
   GLT_STRIDED(LD_F32, LD_F32, float, EPI_STORE, false)
   GLT_STRIDED(LD_F32, LD_F32, float, EPI_RESID, false)

@@ -10,6 +10,10 @@
  * bf16 values are passed as their 16-bit patterns (uint16_t storage).
  * All matrices are row-major. "[R,C]" means R rows of C contiguous elements.
  *
+ * A token's outputs (MLP forward and dx, layer, logits) depend on that token
+ * (attention: its sequence) alone: the same bits whatever other tokens the call
+ * holds.
+ *
  * The reference implements this path as an internal C++ API with shapes held
  * in a process-global config (reference src/config.hpp:40-95, g_cfg). Here the
  * shapes travel in descriptors instead. Citations name the reference function

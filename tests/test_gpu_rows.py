@@ -66,6 +66,38 @@ def test_head(dev, V, D):
             assert torch.equal(_bits(ops.lm_head_bwd(gr[:M].contiguous(), w)), _bits(dx[:M])), M
 
 
+@pytest.mark.parametrize("D,I,pl,bf16", [
+    (512, 1408, [(1408, 256, 0, 512)], False),
+    (260, 390, [(7, 31, 3, 90), (390, 33, 0, 260)], False),
+    (200, 300, [(300, 40, 0, 200)], True),  # not whole 64-K steps: the strided kernel
+])
+def test_strided_mlp(dev, D, I, pl, bf16):
+    """The f32 path, and bf16 shapes off the fragment layout: from one tile to
+    several 64 x 64 tiles per CU."""
+    import torch
+    from glt_amd import ops
+    N = max([I] + [i0 + s for i0, s, _, _ in pl])
+    wg, wu, wd, sl = make_layer(D, I, N, pl, bf16)
+    dt = torch.bfloat16 if bf16 else torch.float32
+    base = ops.BaseMLP(to_dev(wg, dt), to_dev(wu, dt), to_dev(wd, dt))
+    gs = [ops.GraftSlice(s["i0"], s["s"], s["h0"], s["h"], *(to_dev(s[p], torch.float32) for p in ("gate", "up", "down")))
+          .pack() for s in sl]
+    g = torch.Generator(device="cuda").manual_seed(D)
+    x = torch.randn((8300, D), generator=g, device="cuda").to(dt)
+    dy = torch.randn((8300, D), generator=g, device="cuda").to(dt)
+
+    def run(M):
+        y, gp, up, inter = ops.mlp_forward(base, gs, x[:M].contiguous(), N)
+        dx, _ = ops.mlp_backward(base, gs, x[:M].contiguous(), dy[:M].contiguous(), N, gp, up, inter)
+        return dict(y=y, gate=gp, up=up, inter=inter, dx=dx)
+
+    full = run(8300)
+    for M in MS:
+        part = run(M)
+        for k in full:
+            assert torch.equal(_bits(full[k][:M]), _bits(part[k])), (k, M)
+
+
 def test_eval_hash_of_any_batches(dev):
     """A model's logits over eight sequences, hashed as one batch and as batches
     of three, one and four."""
