@@ -512,8 +512,9 @@ static bool read_once(const GArgs& a, bool dual) {
 
 template <int TI, int TJ, int RB, int NWN, int PA, int PB, typename TO, int MODE, bool DUAL>
 static glt_status launch_small(const GArgs& a, hipStream_t st, const char* label) {
-  // (the non-temporal form only where few rows choose it)
-  if constexpr (TJ * NWN <= 4 && (MODE == EPI_SILU || MODE == EPI_STORE))
+  // (the non-temporal form only where the cost model can come with so much B:
+  // f32 outputs, dX and the head's, are narrow and of 32 x 32 tiles then)
+  if constexpr (MODE == EPI_SILU || (MODE == EPI_STORE && (sizeof(TO) == 2 || TI == 1)))
     if (read_once(a, DUAL)) return launch_small_as<TI, TJ, RB, NWN, PA, PB, TO, MODE, DUAL, true>(a, st, label);
   return launch_small_as<TI, TJ, RB, NWN, PA, PB, TO, MODE, DUAL, false>(a, st, label);
 }

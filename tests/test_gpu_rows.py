@@ -66,10 +66,45 @@ def test_head(dev, V, D):
             assert torch.equal(_bits(ops.lm_head_bwd(gr[:M].contiguous(), w)), _bits(dx[:M])), M
 
 
+@pytest.mark.parametrize("I,M", [(8448, 8), (8448, 48), (8448, 100), (17408, 100)])
+def test_mlp_weights_past_the_cache(dev, I, M):
+    """Gate/up of 138 and 285 MB, and dX's as much, which one row of tiles (32 x
+    32, 64 x 64, 128 x 64 and 128 x 128) loads non-temporally, against 600 tokens,
+    which do not."""
+    import torch
+    from glt_amd import ops
+    D = 4096
+    g = torch.Generator(device="cuda").manual_seed(I)
+    rn = lambda *s: torch.randn(s, generator=g, device="cuda").mul_(0.02).bfloat16()
+    base = ops.BaseMLP(rn(I, D), rn(I, D), rn(D, I))
+    x, dy = rn(600, D).mul_(50), rn(600, D).mul_(50)
+
+    def run(n):
+        _, gp, up, inter = ops.mlp_forward(base, [], x[:n].contiguous(), I)
+        dx, _ = ops.mlp_backward(base, [], x[:n].contiguous(), dy[:n].contiguous(), I, gp, up, inter)
+        return gp, up, inter, dx
+
+    for a, b in zip(run(600), run(M)):
+        assert torch.equal(_bits(a[:M]), _bits(b))
+
+
+@pytest.mark.parametrize("V", [32000, 49152])
+def test_head_weights_past_the_cache(dev, V):
+    """The same of an LM head: 64 x 64 to 128 x 256 tiles."""
+    import torch
+    from glt_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.randn((600, 4096), generator=g, device="cuda").bfloat16()
+    w = torch.randn((V, 4096), generator=g, device="cuda").mul_(0.05).bfloat16()
+    y = ops.lm_head_fwd(x, w)
+    for M in (5, 48, 100):
+        assert torch.equal(_bits(ops.lm_head_fwd(x[:M].contiguous(), w)), _bits(y[:M])), M
+
+
 @pytest.mark.parametrize("D,I,pl,bf16", [
     (512, 1408, [(1408, 256, 0, 512)], False),
     (260, 390, [(7, 31, 3, 90), (390, 33, 0, 260)], False),
-    (200, 300, [(300, 40, 0, 200)], True),  # not whole 64-K steps: the strided kernel
+    (360, 500, [(500, 40, 0, 360)], True),  # not whole 64-K steps: the strided kernel
 ])
 def test_strided_mlp(dev, D, I, pl, bf16):
     """The f32 path, and bf16 shapes off the fragment layout: from one tile to
@@ -89,7 +124,9 @@ def test_strided_mlp(dev, D, I, pl, bf16):
     def run(M):
         y, gp, up, inter = ops.mlp_forward(base, gs, x[:M].contiguous(), N)
         dx, _ = ops.mlp_backward(base, gs, x[:M].contiguous(), dy[:M].contiguous(), N, gp, up, inter)
-        return dict(y=y, gate=gp, up=up, inter=inter, dx=dx)
+        res = dy[:M].clone()
+        ops.mlp_forward(base, gs, x[:M].contiguous(), N, residual=res)
+        return dict(y=y, gate=gp, up=up, inter=inter, dx=dx, residual=res)
 
     full = run(8300)
     for M in MS:
@@ -128,14 +165,15 @@ def test_eval_hash_of_any_batches(dev):
     assert batches([8]) == batches([3, 1, 4]) == batches([1] * 8)
 
 
+@pytest.mark.parametrize("K", [1088, 1090])  # the MFMA path; the strided kernel
 @pytest.mark.parametrize("M", [8, 64, 200, 512])
-def test_infinities_and_nan_stay_in_their_rows(dev, M):
+def test_infinities_and_nan_stay_in_their_rows(dev, M, K):
     """A row of infinities, one of NaN and one of the type's largest values
     leave every other row's bits as they are, and give what f32 sums give."""
     import torch
     from glt_amd import ops
-    K, V = 1088, 4104
-    g = torch.Generator(device="cuda").manual_seed(M)
+    V = 4104
+    g = torch.Generator(device="cuda").manual_seed(M + K)
     x = torch.randn((M, K), generator=g, device="cuda").bfloat16()
     w = torch.randn((V, K), generator=g, device="cuda").mul_(0.05).bfloat16()
     bad = x.clone()
