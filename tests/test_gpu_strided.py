@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("M,S,H", [(1, 1, 1), (31, 33, 5), (64, 32, 64), (65, 97, 130), (513, 36, 260), (40, 1024, 12),
-                                   (2100, 768, 260), (1027, 1030, 34)])
+                                   (2100, 768, 260), (1027, 1030, 34), (3300, 1000, 900), (65, 1800, 1792)])
 def test_graft_gemm_kinds(dev, M, S, H):
     """The six graft GEMMs: every pair of operand orientations, lengths off the
     chunks and pieces, few tiles (many wavefronts per tile) to several 64 x 64
