@@ -272,7 +272,9 @@ __device__ __forceinline__ void chunk_range(int V, int c, int& v0, int& v1) {
 // so the cut sets the threads: about kHashThreads of them, four wavefronts per
 // SIMD (16 chunks per row whatever the rows left half the SIMDs idle at 2048
 // rows: 1.29 ms for the two nibble passes, 0.31 this way, half of that from the
-// eight runs instead of sixteen), between 16 chunks per row and 1024.
+// eight runs instead of sixteen), between 16 chunks per row and 1024. The power of
+// two costs up to 40 % just past a step (V = 32000: 2048 rows 118 us, 2049 154, 3000
+// 188, 4096 255; 16 chunks per row with sixteen runs 420, 421, 419, 435).
 constexpr int64_t kHashThreads = 262144;
 __host__ __device__ inline int hash_shift(int64_t rows) {
   int sh = 4;
