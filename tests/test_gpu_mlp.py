@@ -416,7 +416,7 @@ def test_pipelined_adamw_stream_matches_sequential(dev):
     assert torch.count_nonzero(ref[1]).item() > 0  # the step did update the moments
 
 
-@pytest.mark.parametrize("M,D,I,S,n_slices", [(2048, 1024, 2048, 256, 1),   # weight gradients leave CUs idle
+@pytest.mark.parametrize("M,D,I,S,n_slices", [(2048, 1024, 2048, 256, 1),   # weight gradients on small tiles: not forked
                                                (512, 512, 1024, 128, 0),     # no slices: no weight gradients
                                                (512, 4608, 1024, 256, 1),    # rows past 4096: not forked
                                                (1000, 1088, 1024, 128, 1)])  # 136 chunks per row: ragged lanes, ragged M
@@ -462,8 +462,10 @@ def test_mlp_rmsnorm_bwd_equals_the_two_calls(dev, M, D, I, S, n_slices):
 
 
 def test_mlp_rmsnorm_bwd_in_a_graph(dev):
-    """glt_mlp_rmsnorm_bwd's fork onto the helper stream and its join are
-    captured with the caller's stream: a graph of the call, replayed three
+    """glt_mlp_rmsnorm_bwd under capture where the norm's backward follows on the
+    caller's stream (the fork onto the helper stream and its join:
+    test_mlp_rmsnorm_bwd_forks_beside_the_persistent_kernel): a graph of the
+    call, replayed three
     times with eager work between the replays, reproduces the eager call's dx,
     gradients and norm gradient bit for bit every time."""
     import ctypes
