@@ -465,9 +465,8 @@ def test_mlp_rmsnorm_bwd_in_a_graph(dev):
     """glt_mlp_rmsnorm_bwd under capture where the norm's backward follows on the
     caller's stream (the fork onto the helper stream and its join:
     test_mlp_rmsnorm_bwd_forks_beside_the_persistent_kernel): a graph of the
-    call, replayed three
-    times with eager work between the replays, reproduces the eager call's dx,
-    gradients and norm gradient bit for bit every time."""
+    call, replayed three times with eager work between the replays, reproduces
+    the eager call's dx, gradients and norm gradient bit for bit every time."""
     import ctypes
     import torch
     from glt_amd import _ffi as F, ops, synth
@@ -582,6 +581,12 @@ def test_mlp_rmsnorm_bwd_forks_beside_the_persistent_kernel(dev, M, D, S):
     check("profiled")
     call()
     check("eager")
+    # in place: the norm's gradient over its input gradient
+    F.call("glt_mlp_rmsnorm_bwd", ctypes.byref(d), ctypes.byref(b), p(x), p(dy), p(gp), p(up), p(inter), p(dx),
+           garr, p(ws), nbytes, p(x_raw), p(gamma), p(var), 1e-5,
+           p(dx), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    assert torch.equal(dx, nd0)
     s = torch.cuda.Stream()
     s.wait_stream(torch.cuda.current_stream())
     graph = torch.cuda.CUDAGraph()
